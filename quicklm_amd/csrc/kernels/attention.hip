@@ -28,6 +28,8 @@
 
 #include <mutex>
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace {
@@ -471,7 +473,8 @@ __global__ __launch_bounds__(kCombineThreads) void k_attn_combine(
 #pragma unroll
             for (int k = 0; k < KB; ++k) {
                 const int c = cg + NG * (k0 + k);
-                const float f = c < nt ? fs[c] : 0.0f;
+                if (c >= nt) break;  // (a zero weight would make NaN of an infinite record)
+                const float f = fs[c];
                 o.x = fmaf(f, ov[k].x, o.x);
                 o.y = fmaf(f, ov[k].y, o.y);
                 o.z = fmaf(f, ov[k].z, o.z);
@@ -583,10 +586,476 @@ __global__ __launch_bounds__(kThreads) void k_gqa_prep_rows(
     }
 }
 
-// ---- prefill attention, head_dim 128, fp32 cache, on the fp32 matrix cores ----
+// ---- prefill attention, head_dim 128, fp32 cache, on the bf16 matrix cores ----
 //
-// One launch per prefill pass, causal, no per-chunk records and no merge: a
-// workgroup owns 16 consecutive prompt rows and one kv head, wave w the query
+// Causal attention of T prompt rows (attention.cpp:54-82 per row: the scores
+// q . k / sqrt(hd), softmax, the weighted sum of V). The fp32 operands are
+// split exactly into three bf16 terms, x = h + m + l (24 significand bits),
+// and each product takes the six term products down to 2^-18 of the largest
+// (h h, h m, m h, m m, h l, l h; the dropped ones are below 2^-26), summed in
+// fp32 on v_mfma_f32_16x16x32_bf16: 2.7x the fp32 matrix cores' rate
+// (16x16x4). Relative error against 64 bits, 2047 rows of 16 / 4 heads:
+// 2.8e-7 (fp32 matrix cores, 16 keys at a time: 4.5e-7).
+//
+// Bound by the matrix cores and the vector ALUs in turn (the waves of a
+// workgroup are at the products, then at the softmax, together): 2047 rows
+// 131 us at ~35% of the bf16 peak counting all six products, 2048 rows after
+// 2048 keys 300 us. The fp32 form, one 16-row tile a workgroup, took 363 and
+// 787 us: 16x the matrix time a product, its longest tile alone 128 or 256
+// steps of 16 keys; 5 rows after 600 keys 71 us, now 13 and a 4 us merge.
+//
+// Row tiles of 16 are paired first with last (tile a with nt - 1 - a), so
+// every slot of two tiles attends to about the same number of keys. A
+// workgroup is G heads of one kv head x RG slots x NK key blocks of 32: the
+// waves of a slot and head split each staged block of 32 NK keys, keep an
+// online softmax of their own and meet through LDS at the end. Keys are
+// staged split: a thread loads fp32 rows one block ahead, splits them and
+// writes the planes in operand order, so that every matrix operand is one
+// 16-byte LDS read a lane and is used by both row tiles of the wave.
+//   S^T = K Q^T: A = 16 keys (lane: key l % 16, elements 8 (l / 16) .. + 7 of
+//     a 32-element step), B = the tile's Q rows the same way; lane (qd, n)
+//     then holds the scores of row n for keys 4 qd + i of each 16-key half;
+//   O^T += V^T P^T: the k-slots of lane group qd are its own eight keys
+//     (4 qd + i and 16 + 4 qd + i), so the probabilities, split in the
+//     registers that computed them, are the B operand; V is staged for that
+//     order, 8 keys of one column a lane.
+// Lane (qd, n) ends with row n's outputs 16 c + 4 qd .. + 3 for c = 0..7.
+// Keys past the workgroup's last position are clamped to it (probability 0;
+// the cache beyond is not written yet). A value that is not finite goes whole
+// into the l term, which only meets the other side's h, so it acts as it
+// would in an fp32 product.
+// gridDim.z > 1 splits the keys in ranges of `ch` and leaves k_attn's record
+// [m, l, -, -, o] per (row, head, range) for k_attn_combine: a few rows over
+// a long context would otherwise walk it on a handful of workgroups.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned pf_u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 pf_bf16x8 __attribute__((ext_vector_type(8)));
+
+// maximum / sum over lanes l, l ^ 16, l ^ 32, l ^ 48 (the four lane groups of
+// a 16-lane column), on lane swaps instead of LDS permutes
+__device__ __forceinline__ float cols_max(float v) { return xor32_max(xor16_max(v)); }
+__device__ __forceinline__ float cols_sum(float v) { return xor32_add(xor16_add(v)); }
+
+struct Split8 {
+    pf_u32x4 t[3];  // h, m, l: eight bf16 each
+};
+
+// eight floats, finite and below the largest bf16, as three bf16 terms (exact)
+__device__ __forceinline__ Split8 split8_finite(const float (&x)[8]) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    Split8 s;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const f32x2 v = {a, b};
+            const unsigned w = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+            s.t[k][i] = w;
+            a -= __uint_as_float(w << 16);
+            b -= __uint_as_float(w & 0xffff0000u);
+        }
+    }
+    return s;
+}
+
+// the same for any floats: one that is not finite, or would round to
+// infinity, is left whole (truncated to bf16) in the l term
+__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+    Split8 s = split8_finite(x);
+    unsigned top = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) top = max(top, __float_as_uint(x[i]) & 0x7fffffffu);
+    if (__builtin_expect(top >= 0x7f7f8000u, 0)) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const unsigned u = __float_as_uint(x[i]), a = u & 0x7fffffffu;
+            const unsigned half = 0xffffu << (16 * (i & 1));
+            const unsigned whole = (u >> 16) | (a > 0x7f800000u ? 0x40u : 0u);
+            if (a >= 0x7f7f8000u) {
+                s.t[0][i / 2] &= ~half;
+                s.t[1][i / 2] &= ~half;
+                s.t[2][i / 2] = (s.t[2][i / 2] & ~half) | (whole << (16 * (i & 1)));
+            }
+        }
+    }
+    return s;
+}
+
+__device__ __forceinline__ f32x4 mfma_bf16(pf_u32x4 a, pf_u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pf_bf16x8, a),
+                                                   __builtin_bit_cast(pf_bf16x8, b), c, 0, 0, 0);
+}
+
+// the term products of one 32-deep step below h h, small ones first
+#define QLM_PF_SMALL_TERMS(STEP) STEP(0, 2) STEP(2, 0) STEP(1, 1) STEP(0, 1) STEP(1, 0)
+
+// 2^x for x <= 0 by v_exp_f32 (1 ulp)
+__device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+template <int G>
+struct PfShape {
+    static constexpr int RG = G >= 4 ? 1 : 4 / G;  // slots (pairs of row tiles) a workgroup
+    static constexpr int NK = G == 8 ? 1 : 2;      // 32-key blocks staged at a time
+    static constexpr int NTH = G * RG * NK * QLM_WAVE;
+};
+
+// Operand order of one 32-key block of a kv head, in 16-byte units: K [term
+// 3][octet of elements 16][key 32], V [term 3][lane group 4][column 128] (the
+// eight keys of lane group qd in its k-slot order).
+constexpr int kPfUnits = 3 * 512;  // units of a block's K or V
+
+__device__ __forceinline__ int pf_v_key(int qd, int j) { return 4 * qd + (j & 3) + 4 * (j & 4); }
+
+// The blocks of every kv head, split once for all workgroups of k_attn_pf
+// (each of which would split all keys again): planes[(g * blocks + b) * 2 *
+// kPfUnits]: K units, then V units. Keys past the last repeat it.
+__global__ __launch_bounds__(256) void k_pf_split(const float* __restrict__ kc,
+                                                  const float* __restrict__ vc, int n_kv, int keys,
+                                                  pf_u32x4* __restrict__ planes) {
+    const int b = blockIdx.x, g = blockIdx.y, lim = keys - 1 - 32 * b;
+    const unsigned kstride = (unsigned)n_kv * 128;
+    const float* kp = kc + (size_t)32 * b * kstride + (size_t)g * 128;
+    const float* vp = vc + (size_t)32 * b * kstride + (size_t)g * 128;
+    pf_u32x4* dst = planes + ((size_t)g * gridDim.x + b) * 2 * kPfUnits;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = threadIdx.x + 256 * u;
+        const float* kr = kp + ((unsigned)min(i & 31, lim) * kstride + 8u * (i >> 5));
+        const float4 a = *reinterpret_cast<const float4*>(kr);
+        const float4 c = *reinterpret_cast<const float4*>(kr + 4);
+        const float kx[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+        float vx[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            vx[j] = vp[(unsigned)min(pf_v_key(i >> 7, j), lim) * kstride + (unsigned)(i & 127)];
+        const Split8 ka = split8(kx), va = split8(vx);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            dst[512 * t + i] = ka.t[t];
+            dst[kPfUnits + 512 * t + i] = va.t[t];
+        }
+    }
+}
+
+// PRE: the planes of k_pf_split are staged as they are, the next K blocks
+// requested before the P.V product and the V blocks before the scores; else
+// each workgroup splits its keys itself.
+template <int G, bool PRE>
+__global__ __launch_bounds__(PfShape<G>::NTH, 2) void k_attn_pf(
+    const float* __restrict__ qkv, int ldq, int qhs, const float* __restrict__ kc,
+    const float* __restrict__ vc, const pf_u32x4* __restrict__ planes, int n_kv, int p0, int T,
+    int gated, float* __restrict__ out, int ldo, float qscale, int ch, float* __restrict__ work) {
+    constexpr int HD = 128, RG = PfShape<G>::RG, NK = PfShape<G>::NK, NTH = PfShape<G>::NTH;
+    // units between a staged K plane's octets: one more than its 32 keys where
+    // a thread writes 16 octets of a key (they would meet in the same banks)
+    constexpr int KST = PRE ? 32 : 33, KB = 3 * 16 * KST;
+    constexpr int NU = NK * 512 / NTH;  // octets (K) and 8-key columns (V) a thread stages
+    __shared__ __align__(16) pf_u32x4 ks[NK * KB];
+    __shared__ __align__(16) pf_u32x4 vs[NK * kPfUnits];
+    const int tid = threadIdx.x, lane = tid & (QLM_WAVE - 1);
+    const int w = __builtin_amdgcn_readfirstlane(tid / QLM_WAVE);
+    const int g = blockIdx.y, kb = w / (G * RG), rg = (w / G) % RG, h = g * G + w % G;
+    const int qd = lane >> 4, n = lane & 15;
+    const int nt = (T + 15) / 16, slots = (nt + 1) / 2;
+    const int slot0 = blockIdx.x * RG;  // the workgroup's longest
+    // keys [kbeg, kend) of this workgroup: its range, up to its last row's position
+    const int kbeg = blockIdx.z * ch;
+    const int wg_last = p0 + min(16 * (nt - 1 - slot0) + 15, T - 1);
+    const int kend = min(kbeg + ch, wg_last + 1);
+    if (kbeg >= kend) return;
+    // tile 1 is the slot's later tile, tile 0 its earlier one (absent in a
+    // middle slot of an odd count); a wave past the last slot only stages
+    const int slot = slot0 + rg;
+    int t0[2] = {16 * slot, 16 * (nt - 1 - slot)}, last[2];
+    last[1] = slot < slots ? p0 + min(t0[1] + 15, T - 1) : -1;
+    last[0] = slot < slots && t0[0] < t0[1] ? p0 + t0[0] + 15 : -1;
+
+    // PRE: this thread's units of the NK blocks from key k0, K (0) or V (1)
+    constexpr int PU = kPfUnits / NTH;  // units a thread and block
+    static_assert(PU * NTH == kPfUnits || !PRE, "whole rounds a block");
+    const int nblk = (p0 + T + 31) / 32;
+    const pf_u32x4* pb = planes + (size_t)g * nblk * 2 * kPfUnits;
+    pf_u32x4 px[NK * PU];
+    auto request = [&](int v, int k0) {
+#pragma unroll
+        for (int b = 0; b < NK; ++b) {
+            const pf_u32x4* src = pb + ((size_t)min(k0 / 32 + b, nblk - 1) * 2 + v) * kPfUnits;
+#pragma unroll
+            for (int u = 0; u < PU; ++u) px[b * PU + u] = src[(unsigned)(tid + NTH * u)];
+        }
+    };
+    auto put = [&](pf_u32x4* dst) {
+#pragma unroll
+        for (int u = 0; u < NK * PU; ++u) dst[tid + NTH * u] = px[u];
+    };
+    if constexpr (PRE) request(0, kbeg);
+
+    Split8 qf[2][4];
+    int qpos[2];
+    {
+        f32x4 raw[2][4][2];  // every load requested before the first is used
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const int tq = max(0, min(t0[r] + n, T - 1));
+            qpos[r] = p0 + tq;
+            const float* qr = qkv + (size_t)tq * ldq + (size_t)h * qhs + 8 * qd;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                raw[r][s][0] = *reinterpret_cast<const f32x4*>(qr + 32 * s);
+                raw[r][s][1] = *reinterpret_cast<const f32x4*>(qr + 32 * s + 4);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                float x[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = raw[r][s][i >> 2][i & 3] * qscale;
+                qf[r][s] = split8(x);
+            }
+    }
+    f32x4 o[2][8];
+    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};  // l: this lane's keys only
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) o[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // row offsets within a block in 32 bits, the block's base in scalars
+    const unsigned kstride = (unsigned)n_kv * HD;
+    float kx[NU][8], vx[NU][8];
+    auto fetch = [&](int k0) {
+        const size_t at = (size_t)k0 * kstride + (size_t)g * HD;
+        const float* kp = kc + at;
+        const float* vp = vc + at;
+        const int lim = kend - 1 - k0;
+        int tv = tid;  // opaque: the offsets are recomputed, not kept in registers
+        asm volatile("" : "+v"(tv));
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const int i = tv + NTH * u;
+            const float* kr = kp + ((unsigned)min(i >> 4, lim) * kstride + 8u * (i & 15));
+            const float4 a = *reinterpret_cast<const float4*>(kr);
+            const float4 b = *reinterpret_cast<const float4*>(kr + 4);
+            kx[u][0] = a.x, kx[u][1] = a.y, kx[u][2] = a.z, kx[u][3] = a.w;
+            kx[u][4] = b.x, kx[u][5] = b.y, kx[u][6] = b.z, kx[u][7] = b.w;
+            const int key = 32 * (i >> 9), kg = (i >> 7) & 3;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                vx[u][j] = vp[(unsigned)min(key + pf_v_key(kg, j), lim) * kstride +
+                              (unsigned)(i & 127)];
+        }
+    };
+    auto stage = [&]() {
+        int tv = tid;
+        asm volatile("" : "+v"(tv));
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const int i = tv + NTH * u, key = i >> 4;
+            const Split8 a = split8(kx[u]), b = split8(vx[u]);
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                ks[(key >> 5) * KB + (16 * t + (i & 15)) * KST + (key & 31)] = a.t[t];
+                vs[(i >> 9) * kPfUnits + 512 * t + (i & 511)] = b.t[t];
+            }
+        }
+    };
+    // scores of the wave's 32 keys for row tiles R0 .. 1, in units of log2;
+    // the h h products apart from the small ones: 4 roundings at the size of
+    // the score instead of 24
+    f32x4 s[2][2];
+    auto scores = [&](auto first) {
+        constexpr int R0 = decltype(first)::value;
+        f32x4 sl[2][2];
+#pragma unroll
+        for (int r = R0; r < 2; ++r)
+            s[r][0] = s[r][1] = sl[r][0] = sl[r][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st < 4; ++st)
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                pf_u32x4 kf[3];
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    kf[t] = ks[kb * KB + (16 * t + 4 * st + qd) * KST + 16 * half + n];
+#define QLM_PF_S(TK, TQ)               \
+    _Pragma("unroll") for (int r = R0; r < 2; ++r) \
+        sl[r][half] = mfma_bf16(kf[TK], qf[r][st].t[TQ], sl[r][half]);
+                QLM_PF_SMALL_TERMS(QLM_PF_S)
+#undef QLM_PF_S
+#pragma unroll
+                for (int r = R0; r < 2; ++r)
+                    s[r][half] = mfma_bf16(kf[0], qf[r][st].t[0], s[r][half]);
+            }
+#pragma unroll
+        for (int r = R0; r < 2; ++r)
+#pragma unroll
+            for (int half = 0; half < 2; ++half) s[r][half] += sl[r][half];
+    };
+    // their softmax and weighted sum
+    auto weigh = [&](auto first, int k1) {
+        constexpr int R0 = decltype(first)::value;
+        Split8 pf[2];
+#pragma unroll
+        for (int r = R0; r < 2; ++r) {
+            float sc[8], tm = -INFINITY;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) sc[j] = s[r][j >> 2][j & 3];
+            if (k1 + 31 > p0 + t0[r]) {  // some key is past some row (wave-uniform)
+                const int lim = qpos[r] - 4 * qd - k1;
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (16 * (j >> 2) + (j & 3) > lim) sc[j] = -INFINITY;
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) tm = fmaxf(tm, sc[j]);
+            const float mn = fmaxf(m[r], cols_max(tm));
+            // a row that has seen no key yet (all of these masked) stays empty
+            const float mref = mn == -INFINITY ? 0.0f : mn;
+            const float alpha = exp2_fast(m[r] - mref);  // 0 on the first keys
+            float p[8], sum = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                p[j] = exp2_fast(sc[j] - mref);
+                sum += p[j];
+            }
+            l[r] = fmaf(l[r], alpha, sum);
+            m[r] = mn;
+            pf[r] = split8_finite(p);
+            if (__any(alpha != 1.0f)) {  // a maximum moved
+#pragma unroll
+                for (int c = 0; c < 8; ++c) o[r][c] *= alpha;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            pf_u32x4 vf[3];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) vf[t] = vs[kb * kPfUnits + 512 * t + qd * HD + 16 * c + n];
+#define QLM_PF_O(TV, TP)               \
+    _Pragma("unroll") for (int r = R0; r < 2; ++r) \
+        o[r][c] = mfma_bf16(vf[TV], pf[r].t[TP], o[r][c]);
+            QLM_PF_SMALL_TERMS(QLM_PF_O)
+            QLM_PF_O(0, 0)
+#undef QLM_PF_O
+        }
+    };
+
+    constexpr std::integral_constant<int, 0> both{};
+    constexpr std::integral_constant<int, 1> later{};
+    if constexpr (PRE) put(ks);
+    else fetch(kbeg);
+    for (int k0 = kbeg; k0 < kend; k0 += 32 * NK) {
+        const int k1 = k0 + 32 * kb;
+        const bool more = k0 + 32 * NK < kend;
+        // this wave's row tiles: both, the later one, or none
+        const int mode = k1 >= kend || k1 > last[1] ? 2 : k1 > last[0] ? 1 : 0;
+        if constexpr (PRE) request(1, k0);
+        else stage();
+        __syncthreads();  // K is in; PRE: the V of the blocks before is read
+        if constexpr (!PRE)
+            if (more) fetch(k0 + 32 * NK);
+        if (mode == 0) scores(both);
+        if (mode == 1) scores(later);
+        if constexpr (PRE) {
+            put(vs);
+            __syncthreads();  // V is in, K is read
+            if (more) request(0, k0 + 32 * NK);
+        }
+        if (mode == 0) weigh(both, k1);
+        if (mode == 1) weigh(later, k1);
+        if constexpr (PRE) {
+            if (more) put(ks);
+        } else {
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) l[r] = cols_sum(l[r]);
+
+    // ---- the key blocks' waves meet: wave kb = 1 leaves [o | m, l] in LDS,
+    // tile 0 in the K planes and tile 1 in the V planes ----
+    if constexpr (NK > 1) {
+        static_assert(NK == 2, "two key blocks");
+        constexpr int RS = 33;  // floats a lane, odd: conflict-free
+        static_assert(G * RG * QLM_WAVE * (RS + 2) <= 4 * NK * kPfUnits, "fits the planes");
+        __syncthreads();
+        const int at = (w % (G * RG)) * QLM_WAVE + lane;
+        float* mg[2] = {reinterpret_cast<float*>(ks), reinterpret_cast<float*>(vs)};
+        constexpr int ML = G * RG * QLM_WAVE * RS;
+        if (kb == 1) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+#pragma unroll
+                for (int c = 0; c < 32; ++c) mg[r][at * RS + c] = o[r][c >> 2][c & 3];
+                mg[r][ML + 2 * at] = m[r];
+                mg[r][ML + 2 * at + 1] = l[r];
+            }
+        }
+        __syncthreads();
+        if (kb == 1) return;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const float m1 = mg[r][ML + 2 * at], l1 = mg[r][ML + 2 * at + 1];
+            const float mn = fmaxf(m[r], m1), mref = mn == -INFINITY ? 0.0f : mn;
+            const float f0 = exp2_fast(m[r] - mref), f1 = exp2_fast(m1 - mref);
+            l[r] = l[r] * f0 + l1 * f1;
+            m[r] = mn;
+#pragma unroll
+            for (int c = 0; c < 32; ++c)
+                o[r][c >> 2][c & 3] = o[r][c >> 2][c & 3] * f0 + mg[r][at * RS + c] * f1;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int tq = t0[r] + n;
+        if (last[r] < kbeg || tq >= T) continue;
+        if (work) {
+            // the record's maximum is in natural units; what its rounding
+            // changes goes into l and o
+            const float mr = m[r] * 0.69314718f;
+            float e = fmaf(-mr, 1.44269502f, m[r]);
+            e = m[r] == -INFINITY ? 0.0f : fmaf(-mr, 1.92596303e-8f, e);
+            const float f = exp2_fast(e);
+            float* rec = work + (((size_t)tq * (gridDim.y * G) + h) * gridDim.z + blockIdx.z) *
+                                    (HD + 4);
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                *reinterpret_cast<f32x4*>(rec + 4 + 16 * c + 4 * qd) = o[r][c] * f;
+            if (qd == 0) {
+                rec[0] = mr;
+                rec[1] = l[r] * f;
+            }
+            continue;
+        }
+        const float* grow = qkv + (size_t)tq * ldq + (size_t)h * qhs + HD;
+        float* dst = out + (size_t)tq * ldo + (size_t)h * HD;
+        const float inv = 1.0f / l[r];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const int e = 16 * c + 4 * qd;
+            f32x4 y = o[r][c] * inv;
+            if (gated) {
+                const f32x4 gg = *reinterpret_cast<const f32x4*>(grow + e);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[i] /= 1.0f + expf(-gg[i]);
+            }
+            *reinterpret_cast<f32x4*>(dst + e) = y;
+        }
+    }
+}
+#undef QLM_PF_SMALL_TERMS
+
+// ---- the same over few keys, on the fp32 matrix cores ----
+//
+// For launches of at most kPfFewKeys keys, where k_attn_pf's splits, merge
+// and larger code cost more than its products save (with the rows'
+// preparation: 64 rows 19 against 24 us, 160 rows 30.5 against 32.6, 256 rows
+// 41 against 38): a workgroup owns 16 consecutive prompt rows and one kv head, wave w the query
 // head g G + w, and walks the keys 0 .. (its last row's position) in tiles of
 // 16 with an online softmax per row (attention.cpp:54-82 per row: the scores
 // q . k / sqrt(hd), softmax, the weighted sum of V). Both products run on
@@ -602,29 +1071,8 @@ __global__ __launch_bounds__(kThreads) void k_gqa_prep_rows(
 // Lane (qd, n) ends with row n's outputs 16 c + 4 qd .. + 3 for c = 0..7.
 // Key rows past the tile's last position are clamped to it (their
 // probabilities are 0 and the cache beyond is not written yet).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// maximum / sum over lanes l, l ^ 16, l ^ 32, l ^ 48 (the four lane groups of
-// a 16-lane column), on lane swaps instead of LDS permutes
-__device__ __forceinline__ float cols_max(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                    false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                    false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float cols_sum(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                    false);
-    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
-                                                    false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 template <int G>
-__global__ __launch_bounds__(G * QLM_WAVE) void k_attn_pf(const float* __restrict__ qkv, int ldq,
+__global__ __launch_bounds__(G * QLM_WAVE) void k_attn_pf_few(const float* __restrict__ qkv, int ldq,
                                                           int qhs, const float* __restrict__ kc,
                                                           const float* __restrict__ vc, int n_kv,
                                                           int p0, int T, int gated,
@@ -997,6 +1445,8 @@ constexpr int kNtModel = 1;  // decode step: one sub-tile per chunk (many short 
 constexpr int kNtLong = 4;   // isolated API: contexts up to 32k
 
 constexpr int kPrefillSlice = 256;  // query rows per prefill attention launch
+constexpr int kPfFewKeys = 192;     // keys up to which k_attn_pf_few takes a prefill
+constexpr int kPfPlaneRows = 256;   // rows from which k_attn_pf's keys are split beforehand
 
 int chunk_len(int hd, int nt) { return (hd == 128 ? 64 : 32) * nt; }
 int nchunks_for(int max_seq, int ch) { return (max_seq + ch - 1) / ch; }
@@ -1319,6 +1769,41 @@ extern "C" int qlm_attention_decode_noalloc(const float* q, const void* k_cache,
                             w, p, as_stream(stream));
 }
 
+namespace {
+
+// Launch of the prefill attention (k_attn_pf). Key ranges: one, unless the
+// launch would leave most of the chip idle; then as many as bring it to ~256
+// workgroups, at least 64 keys each, and no more records than the workspace
+// holds. Split planes (k_pf_split): for G >= 4 and enough rows, where the
+// workspace has room for them before the records.
+struct PfPlan {
+    int groups, ranges, ch;
+    bool planes;
+    size_t rec_at;  // floats from the workspace's start to the records
+};
+PfPlan prefill_plan(int G, int n_q, int n_kv, int p0, int T, int max_seq) {
+    const int rg = G >= 4 ? 1 : 4 / G;
+    const int slots = ((T + 15) / 16 + 1) / 2;
+    PfPlan p;
+    p.groups = (slots + rg - 1) / rg;
+    const int keys = p0 + T;
+    const size_t bytes = records_bytes(kPrefillSlice, n_q, 128, max_seq, kNtLong);
+    const size_t row = (size_t)n_q * (128 + 4) * sizeof(float);  // a row's records, one range
+    const size_t pl = (size_t)n_kv * ((keys + 31) / 32) * 2 * kPfUnits * 16;
+    int z = 256 / (p.groups * n_kv);
+    z = z < keys / 64 ? z : keys / 64;
+    const size_t room = bytes / (row * T);
+    z = (size_t)z < room ? z : (int)room;
+    if (z < 1) z = 1;
+    p.ch = ((keys + z - 1) / z + 63) / 64 * 64;
+    p.ranges = (keys + p.ch - 1) / p.ch;
+    p.planes = G >= 4 && T >= kPfPlaneRows && pl + (p.ranges > 1 ? row * T * p.ranges : 0) <= bytes;
+    p.rec_at = p.planes ? pl / sizeof(float) : 0;
+    return p;
+}
+
+}  // namespace
+
 extern "C" size_t qlm_gqa_prefill_workspace_bytes(int n_q, int hd, int max_seq) {
     if (n_q <= 0 || hd <= 0 || max_seq <= 0) return 0;
     return records_bytes(kPrefillSlice, n_q, hd, max_seq, kNtLong);
@@ -1355,19 +1840,51 @@ extern "C" int qlm_gqa_prefill(float* qkv, int ldqkv, const float* q_norm, const
     int rc = qlm_launch_status();
     if (rc != QLM_OK) return rc;
     if (hd == 128 && (ldqkv % 4) == 0 && (ldo % 4) == 0 && (qstride % 4) == 0) {
-        const dim3 grid((T + 15) / 16, n_kv);
-        const float scale = 1.0f / sqrtf(128.0f);
-#define QLM_ATTN_PF(GG)                                                                         \
-        if (G == GG) {                                                                          \
-            hipLaunchKernelGGL((k_attn_pf<GG>), grid, dim3(GG * QLM_WAVE), 0, st, qkv, ldqkv,   \
-                               qstride, k_cache, v_cache, n_kv, p0, T, gated, out, ldo, scale); \
-            return qlm_launch_status();                                                         \
+        if (p0 + T <= kPfFewKeys) {
+            const dim3 grid((T + 15) / 16, n_kv);
+            const float scale = 1.0f / sqrtf(128.0f);
+#define QLM_ATTN_FEW(GG)                                                                        \
+            if (G == GG) {                                                                      \
+                hipLaunchKernelGGL((k_attn_pf_few<GG>), grid, dim3(GG * QLM_WAVE), 0, st, qkv,  \
+                                   ldqkv, qstride, k_cache, v_cache, n_kv, p0, T, gated, out,   \
+                                   ldo, scale);                                                 \
+                return qlm_launch_status();                                                     \
+            }
+            QLM_ATTN_FEW(1)
+            QLM_ATTN_FEW(2)
+            QLM_ATTN_FEW(4)
+            QLM_ATTN_FEW(8)
+#undef QLM_ATTN_FEW
         }
-        QLM_ATTN_PF(1)
-        QLM_ATTN_PF(2)
-        QLM_ATTN_PF(4)
-        QLM_ATTN_PF(8)
+        const PfPlan pl = prefill_plan(G, n_q, n_kv, p0, T, max_seq);
+        float* rec = pl.ranges > 1 ? w + pl.rec_at : nullptr;
+        pf_u32x4* planes = reinterpret_cast<pf_u32x4*>(work);
+        if (pl.planes) {
+            hipLaunchKernelGGL(k_pf_split, dim3((p0 + T + 31) / 32, n_kv), dim3(256), 0, st,
+                               k_cache, v_cache, n_kv, p0 + T, planes);
+            rc = qlm_launch_status();
+            if (rc != QLM_OK) return rc;
+        }
+        const dim3 grid(pl.groups, n_kv, pl.ranges);
+        const float qscale = 1.44269504088896341f / sqrtf(128.0f);
+        rc = QLM_ERR_SHAPE;
+#define QLM_ATTN_PF(GG, PRE)                                                                    \
+        if (G == GG && pl.planes == PRE) {                                                      \
+            hipLaunchKernelGGL((k_attn_pf<GG, PRE>), grid, dim3(PfShape<GG>::NTH), 0, st, qkv,  \
+                               ldqkv, qstride, k_cache, v_cache, planes, n_kv, p0, T, gated,    \
+                               out, ldo, qscale, pl.ch, rec);                                   \
+            rc = qlm_launch_status();                                                           \
+        }
+        QLM_ATTN_PF(1, false)
+        QLM_ATTN_PF(2, false)
+        QLM_ATTN_PF(4, false)
+        QLM_ATTN_PF(4, true)
+        QLM_ATTN_PF(8, false)
+        QLM_ATTN_PF(8, true)
 #undef QLM_ATTN_PF
+        if (rc != QLM_OK || !rec) return rc;
+        return launch_combine<128>(rec, pl.ranges, pl.ch, max_seq, nullptr, p0 + 1, 1,
+                                   gated ? qkv : nullptr, ldqkv, qstride, out, ldo, n_q, T, st);
     }
     for (int s0 = 0; s0 < T; s0 += kPrefillSlice) {
         const int rows = T - s0 < kPrefillSlice ? T - s0 : kPrefillSlice;

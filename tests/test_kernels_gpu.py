@@ -793,6 +793,52 @@ def test_gqa_prefill(hip, orc, rng, n_q, n_kv, hd, rot, gated, p0, T):
     assert np.array_equal(dvc.to_numpy(vc.shape, np.float32)[:p0 + T], vref[:p0 + T])
 
 
+@pytest.mark.parametrize("n_q,n_kv,p0,T", [
+    (16, 4, 0, 192), (16, 4, 0, 193),  # the last launch of the few-key form, the first after it
+    (16, 4, 600, 5), (8, 8, 150, 60), (8, 4, 200, 45), (16, 2, 300, 33),  # key ranges merged
+    (16, 4, 70, 290), (16, 2, 0, 272),  # split planes; 19 (a middle tile) and 17 row tiles
+    (8, 4, 1, 255), (8, 8, 3, 400)])    # slots past the last in the last workgroup
+def test_gqa_prefill_split_terms(hip, orc, rng, n_q, n_kv, p0, T):
+    """head_dim 128 over more than a few keys (fp32 operands as three bf16
+    terms): every launch form against the oracle row by row, to the fp32
+    attention's bar, and an infinite V element of a key that every row sees
+    (weighted by probabilities > 0: the output column is infinite)."""
+    hd, rot, max_seq, theta, gated = 128, 32, 700, 1e6, 1
+    ld = n_q * 2 * hd + 2 * n_kv * hd
+    qn = (rng.standard_normal(hd) * 0.02).astype(np.float32)
+    kn = (rng.standard_normal(hd) * 0.02).astype(np.float32)
+    cos_t, sin_t = orc.rope_table(theta, rot, max_seq)
+    kc = np.zeros((max_seq, n_kv, hd), np.float32)
+    vc = np.zeros_like(kc)
+    kc[:p0] = rng.standard_normal((p0, n_kv, hd))
+    vc[:p0] = rng.standard_normal((p0, n_kv, hd))
+    qkv = rng.standard_normal((T, ld)).astype(np.float32)
+    kref, vref = kc.copy(), vc.copy()
+    ref = np.stack([orc.gqa_core(qkv[t].copy(), qn, kn, theta, rot, kref, vref, p0 + t, n_q, n_kv,
+                                 hd, gated) for t in range(T)])
+    nwork = hip.lib().qlm_gqa_prefill_workspace_bytes(n_q, hd, max_seq)
+
+    def run(vcache):
+        work = hip.DeviceBuffer(nwork)
+        work.upload(np.full(nwork, 0x5A, np.uint8))  # no initial contents are required
+        do = hip.DeviceBuffer(T * n_q * hd * 4)
+        say("gqa_prefill split terms", n_q, n_kv, p0, T)
+        hip.call("qlm_gqa_prefill", dev(hip, qkv), ld, dev(hip, qn), dev(hip, kn),
+                 dev(hip, cos_t), dev(hip, sin_t), rot, dev(hip, kc), dev(hip, vcache), max_seq,
+                 p0, T, do, n_q * hd, n_q, n_kv, hd, gated, work, None)
+        return do.to_numpy((T, n_q, hd), np.float32)
+
+    got = run(vc)
+    assert rel_err(got.reshape(T, -1), ref) < 1e-5
+    if p0 > 0:
+        vinf = vc.copy()
+        vinf[0, 0, 7] = -np.inf
+        again, G = run(vinf), n_q // n_kv
+        assert np.all(again[:, :G, 7] == -np.inf)
+        again[:, :G, 7] = got[:, :G, 7]
+        assert np.array_equal(again, got)
+
+
 # ---------------------------------------------------------------- A8/A9 GQA
 @pytest.mark.parametrize("n_q,n_kv,hd,rot,gated,max_seq,start",
                          [(16, 4, 128, 32, 1, 600, (300, 511)),
