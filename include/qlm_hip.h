@@ -186,8 +186,11 @@ int qlm_gemv_mx_l2_plan(const void* q_tiles, const float* s_tiles, int group, in
  * 0: y = x.W^T; 1: y += x.W^T; 2: SwiGLU with weights [2F, K] and N = F
  * outputs. Any M >= 1; K a multiple of 32; G = 32 or K. work: device
  * scratch of qlm_matmul_i8_workspace_bytes(M, N, K, epilogue) bytes (row
- * scales and K-split partial sums; no initial contents needed; calls that
- * share it must be ordered on one stream). */
+ * scales or the split activation, and K-split partial sums; no initial
+ * contents needed; calls that share it must be ordered on one stream). More
+ * than 64 rows split K over workgroups where that fills the GPU; with less
+ * workspace, down to 4 M + 4 M K bytes (each term rounded up to 256), they
+ * take the slices whose sums fit. The size never falls with M. */
 size_t qlm_matmul_i8_workspace_bytes(int M, int N, int K, int epilogue);
 
 int qlm_matmul_i8(const float* x, int ldx, const float* norm_w, float eps, const int8_t* q,
@@ -585,14 +588,16 @@ int qlm_lm_head_greedy_mx4(const float* x, const float* norm_w, float eps,
  * qlm_matmul_w_workspace_bytes(K) bytes when norm_w is given. K a multiple
  * of 16; x, W, norm_w 16-byte aligned. */
 /* bf16 weight rows (no scales) with many activation rows, the prefill form:
- * 128 x 64 output tiles on the bf16 matrix cores, the weights staged through
- * LDS as they are, the activation split into bf16 hi + lo (2^-17 of x), the
- * MFMAs chained over K in fp32. Same arguments and epilogues as
+ * tiles on the bf16 matrix cores, the weights staged through LDS as they are,
+ * the activation split into bf16 hi + lo (2^-17 of x), the MFMAs chained over
+ * K in fp32. Same arguments and epilogues as
  * qlm_matmul_w (which calls it for bf16 weights and M > 16). work: with
  * qlm_matmul_bf16_workspace_bytes(M, K) bytes the activation is split once
- * (RMSNorm applied) into bf16 planes there; with less, each workgroup
- * splits its chunks itself, and then norm_w still needs the first M floats
- * (row scales). K a multiple of 32. */
+ * (RMSNorm applied) into bf16 planes there, and K is split over workgroups
+ * where that fills the GPU (with less, the slices whose sums fit); below 4 M +
+ * 4 M K bytes (each term rounded up to 256) each workgroup splits its chunks
+ * itself, and then norm_w still needs the first M floats (row scales). K a
+ * multiple of 32. */
 size_t qlm_matmul_bf16_workspace_bytes(int M, int K);
 int qlm_matmul_bf16(const float* x, int ldx, const float* norm_w, float eps, const uint16_t* w,
                     float* y, int ldy, int M, int N, int K, int epilogue, void* work,

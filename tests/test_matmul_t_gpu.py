@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 from tests.test_kernels_gpu import _mx_layout, _weights, dev
-from tests.util import rel_err, say
+from tests.util import bf16_bits, rel_err, say
 
 pytestmark = pytest.mark.gpu
 
@@ -330,3 +330,56 @@ def test_matmul_i8_rows64_rounds(hip, orc, rng, M, N, K, epi):
     assert rel_err(dy.to_numpy((M, N), np.float32), ref) < 1e-5
 
 
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (65, 255, 64),     # half a row block, one column short, two groups (one slice)
+    (128, 256, 1088),  # exactly one block; 34 groups in ragged slices
+    (129, 257, 512),   # one row and one column over
+    (257, 385, 2048),  # a 1-row last tile; a wave whose columns all lie past N
+])
+@pytest.mark.parametrize("epi", ["store", "store_norm", "resid", "swiglu_norm"])
+@pytest.mark.parametrize("form", ["g32", "row", "bf16"])
+def test_matmul_many_rows_edges(hip, orc, rng, M, N, K, epi, form):
+    """The many-row matmul at the edges of its 128 x 256 blocks, whole and in K
+    slices (the full workspace) and whole (the least workspace), over tile-major
+    and row-major int8 and bf16 rows. Bar against the fp32 oracle: the
+    activation's hi + lo split leaves 2^-17 of a value and the fp32 sums
+    sqrt(K) 2^-24 of the result, below 1e-5 normwise; 5e-5 for bf16 rows, whose
+    oracle sums in another order."""
+    e = EPI[epi]
+    rows_w = 2 * N if epi.startswith("swiglu") else N
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    nw = (rng.standard_normal(K) * 0.02).astype(np.float32)
+    ldy = N + 3
+    y0 = rng.standard_normal((M, ldy)).astype(np.float32)
+    xin = orc.rms_norm(x, nw, 1e-6) if epi.endswith("norm") else x
+    if form == "bf16":
+        w = bf16_bits((rng.standard_normal((rows_w, K)) * 0.05).astype(np.float32))
+        lg = orc.matmul_w(xin, w)
+        full = hip.lib().qlm_matmul_bf16_workspace_bytes(M, K)
+        dw = dev(hip, w)
+        runs = [("qlm_matmul_bf16", (dw,))]
+    else:
+        g = 32 if form == "g32" else K
+        q, s = _weights(orc, rng, rows_w, K, g)
+        lg = orc.matmul_i8(xin, q, s, g)
+        dq, ds, keep = _mx_layout(hip, q, s, g, N, K, rows_w // N)
+        full = hip.lib().qlm_matmul_i8_workspace_bytes(M, N, K, e)
+        runs = [("qlm_matmul_i8", (keep[0], keep[1], g)), ("qlm_matmul_i8_tm", (dq, ds, g))]
+    ref = (y0[:, :N] + lg if epi == "resid" else lg if epi.startswith("store")
+           else orc.silu_mul(lg[:, :N].copy(), lg[:, N:].copy()))
+    least = sum((b + 255) // 256 * 256 for b in (4 * M, 4 * M * K))
+    work = hip.DeviceBuffer(full)
+    dx, dnw = dev(hip, x), dev(hip, nw) if epi.endswith("norm") else None
+    for nbytes in (full, least):
+        outs = []
+        for fn, args in runs:
+            work.upload(np.full(full, 0xA5, np.uint8))
+            dy = dev(hip, y0)
+            say(fn, form, epi, M, N, K, nbytes)
+            hip.call(fn, dx, K, dnw, 1e-6, *args, dy, ldy, M, N, K, e, work, nbytes, None)
+            outs.append(dy.to_numpy((M, ldy), np.float32))
+            assert np.array_equal(outs[-1][:, N:], y0[:, N:])
+            assert rel_err(outs[-1][:, :N], ref) < (5e-5 if form == "bf16" else 1e-5)
+        assert all(np.array_equal(o, outs[0]) for o in outs)
