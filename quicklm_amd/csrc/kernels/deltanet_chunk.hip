@@ -19,15 +19,24 @@
 //   k_dn_chunk_prep   per (16 rows, head): conv taps from the prompt rows or
 //                     the ring (positions before p0), SiLU, L2 norms, gates --
 //                     the decode step's arithmetic;
-//   k_dn_chunk_intra  per (chunk, head): K K^T and the masked, decayed Q K^T
-//                     on the matrix cores, the triangular solve for T (one
-//                     column per lane, unrolled), U and Wk on the matrix cores;
-//   k_dn_chunk_inter  per (head, 16 value columns): chunks in order; W and
-//                     the state update on the matrix cores, the state slice
-//                     living in the accumulators, and on other waves O of
-//                     the chunk before;
-//   k_dn_chunk_post   per (16 rows, head): head RMSNorm + SiLU(z) gate (decode
+//   k_dn_chunk_intra  per (chunk, head): everything that does not depend on
+//                     the state: the masked, decayed K K^T and Q K^T, the
+//                     inverse (I + A)^-1 by blocks of 16, U, Wk and the decayed
+//                     K^T;
+//   k_dn_chunk_chain  per (head, 16 value columns): chunks in order, W and the
+//                     state only;
+//   k_dn_chunk_out    per (chunk, head): the outputs from the states and W of
+//                     all chunks at once, head RMSNorm + SiLU(z) gate (decode
 //                     arithmetic) and the conv ring rows of the last positions.
+//
+// Operand order. A 16x16 block feeds or leaves a matrix instruction as one
+// float4 a lane: lane (l16, l4) holds its elements (l16, 4 l4 .. + 3), rows
+// first as the A operand and columns first as the B operand, where the K
+// index of product j of a block is 4 l4 + j; a result D holds (rows 4 l4 + i,
+// column l16), which is the B operand's order of the same matrix and the A
+// operand's of its transpose. So every matrix that one kernel hands to the
+// next is stored block by block, 1 KB each, lane after lane, and a product's
+// result is the next product's operand without a transposition.
 
 #include "common.hpp"
 
@@ -39,16 +48,8 @@ constexpr int kD = 128;      // head dim (d_k = d_v)
 constexpr int kC = 64;       // chunk rows
 constexpr int KP = kD + 4;   // padded LDS row of a [64][128] tile
 constexpr int TP = kC + 4;   // padded LDS row of a [64][64] tile
-constexpr int CB = 16;       // value columns per inter-chunk workgroup
-
-// Makes the compiler wait here for the load that produced v.
-__device__ __forceinline__ void landed(float v) { asm volatile("" ::"v"(v)); }
-__device__ __forceinline__ void landed(const float4& v) {
-    landed(v.x);
-    landed(v.y);
-    landed(v.z);
-    landed(v.w);
-}
+constexpr int CB = 16;       // value columns per chain workgroup
+constexpr int kBlk = 256;    // floats of a 16x16 block in operand order
 
 // D += A B on a 16x16 tile, K = 4: lane l supplies A[l%16][l/16] and
 // B[l/16][l%16]; it holds D[(l/16)*4 + i][l%16].
@@ -56,7 +57,22 @@ __device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ size_t rix(int t, int h, int H) { return ((size_t)t * H + h) * kD; }
+// Four products of one block pair: K = 16.
+__device__ __forceinline__ f32x4 mma4(f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = mma(a[j], b[j], c);
+    return c;
+}
+
+__device__ __forceinline__ f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ void st4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
+
+// q, k, v and gate rows are kept by chunk and head: row t of head h is row
+// t % kC of tile (t / kC, h).
+__device__ __forceinline__ size_t gix(int t, int h, int H) {
+    return ((size_t)(t / kC) * H + h) * kC + t % kC;
+}
+__device__ __forceinline__ size_t rix(int t, int h, int H) { return gix(t, h, H) * kD; }
 
 // Rows a prep or post workgroup handles (a conv window slides down them).
 constexpr int kPR = 16;
@@ -114,8 +130,8 @@ __global__ __launch_bounds__(3 * kD) void k_dn_chunk_prep(
         const float* pr = proj + (size_t)t * ldp;
         const float dt = pr[4 * HD + H + h] + dt_bias[h];
         const float sp = dt > 20.0f ? dt : log1pf(expf(dt));
-        alpha[(size_t)t * H + h] = -expf(A_log[h]) * sp;
-        beta[(size_t)t * H + h] = 1.0f / (1.0f + expf(-pr[4 * HD + h]));
+        alpha[gix(t, h, H)] = -expf(A_log[h]) * sp;
+        beta[gix(t, h, H)] = 1.0f / (1.0f + expf(-pr[4 * HD + h]));
     }
     __syncthreads();
     for (int i = wave; i < 2 * kPR; i += 3 * kD / 64) {
@@ -131,464 +147,465 @@ __global__ __launch_bounds__(3 * kD) void k_dn_chunk_prep(
     }
 }
 
-// Global operands that feed the matrix cores straight from registers (the
-// wave's q rows for Q K^T, its 32 value columns for U = T V) are loaded at
-// the start, so their latency passes under the K staging, K K^T and the
-// solve instead of stalling each product step.
+// What a chunk's state-independent part is bound by is the fp32 matrix cores
+// and the latency of its steps in turn, at two workgroups a CU. The products
+// above the diagonal are left out (K K^T, Q K^T, U and Wk: 10 of 16 blocks),
+// and the inverse goes by blocks: each wave inverts one diagonal block (a
+// column a lane, 16 steps), then
+//   [X0 0; -X1 L X0, X1] joins blocks to 32 and to 64 rows,
+// whose two products chain in registers. kk: the chunk's k rows in, the
+// decayed K^T out (all rows are in LDS before the first is overwritten).
 __global__ __launch_bounds__(256, 2) void k_dn_chunk_intra(
-    const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ vv,
+    const float* __restrict__ qn, float* kk, const float* __restrict__ vv,
     const float* __restrict__ alpha, const float* __restrict__ beta, int T, int H,
     float* __restrict__ U, float* __restrict__ Wk, float* __restrict__ Mq,
     float* __restrict__ Gc) {
     __shared__ __attribute__((aligned(16))) float Ks[kC * KP];
-    __shared__ float Ts[kC * TP];
-    __shared__ float gs[kC], bs[kC], gam[kC];
+    __shared__ __attribute__((aligned(16))) float Ts[kC * TP];  // A
+    __shared__ __attribute__((aligned(16))) float Xs[kC * TP];  // (I + A)^-1
+    __shared__ __attribute__((aligned(16))) float gs[kC], bs[kC], bg[kC], dec[kC];
     const int c = blockIdx.x, h = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, l4 = lane >> 4;
-    const int t0 = c * kC;
-    const int nt = min(kC, T - t0);
-    auto row = [&](int t) { return rix(t0 + min(t, nt - 1), h, H); };  // clamped; masked at use
+    const int nt = min(kC, T - c * kC);
+    const size_t tile = (size_t)c * H + h;
+    const size_t base = tile * kC * kD;
 
-    // q[tq][k0 + l4] for k0 = 0, 4, .., 124 (rows of Q K^T)
+    // operands of later products that come straight from memory, requested
+    // first: q rows of this wave's row block, v's 32 columns of this wave
+    // (rows past the last are read as the last and masked at use)
     const int tq = wave * 16 + l16;
-    float qv[kD / 4];
-    {
-        const float* qrow = qn + row(tq);
+    f32x4 qv[kD / 16];
 #pragma unroll
-        for (int i = 0; i < kD / 4; ++i) qv[i] = qrow[4 * i + l4];
-    }
-    // V[k0 + l4][32 wave + 16 ct + l16] for k0 = 0, 4, .., 60 (columns of U)
-    float vr[kC / 4][2];
+    for (int kb = 0; kb < kD / 16; ++kb)
+        qv[kb] = ld4(qn + base + (size_t)min(tq, nt - 1) * kD + 16 * kb + 4 * l4);
+    float vr[kC / 16][4][2];
 #pragma unroll
-    for (int i = 0; i < kC / 4; ++i) {
-        const float* vrow = vv + row(4 * i + l4) + 32 * wave + l16;
-        vr[i][0] = vrow[0];
-        vr[i][1] = vrow[16];
-    }
-    for (int i = tid; i < kC * (kD / 4); i += 256) {
-        const int r = i / (kD / 4), c4 = i % (kD / 4);
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (r < nt) v = *reinterpret_cast<const float4*>(kn + rix(t0 + r, h, H) + c4 * 4);
-        *reinterpret_cast<float4*>(&Ks[r * KP + c4 * 4]) = v;
-    }
-    if (tid < kC) {
-        gs[tid] = tid < nt ? alpha[(size_t)(t0 + tid) * H + h] : 0.0f;
-        bs[tid] = tid < nt ? beta[(size_t)(t0 + tid) * H + h] : 0.0f;
-    }
-    __syncthreads();
-    if (tid == 0) {  // cumulative log-decay, in row order
-        float a = 0.0f;
-        for (int t = 0; t < kC; ++t) {
-            a += gs[t];
-            gs[t] = a;
+    for (int kb = 0; kb < kC / 16; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float* vrow =
+                vv + base + (size_t)min(16 * kb + 4 * l4 + j, nt - 1) * kD + 32 * wave + l16;
+            vr[kb][j][0] = vrow[0];
+            vr[kb][j][1] = vrow[16];
         }
+#pragma unroll
+    for (int n = 0; n < kC * kD / 4 / 256; ++n) {
+        const int i = tid + 256 * n, r = i / (kD / 4), c4 = i % (kD / 4);
+        const f32x4 v = ld4(kk + base + (size_t)min(r, nt - 1) * kD + c4 * 4);
+        st4(&Ks[r * KP + c4 * 4], r < nt ? v : f32x4{0.f, 0.f, 0.f, 0.f});
+    }
+    if (wave == 0) {  // cumulative log-decay and the factors formed from it
+        const size_t g = tile * kC;
+        const int r = min(lane, nt - 1);
+        const float al = alpha[g + r], be = beta[g + r];
+        float a = lane < nt ? al : 0.0f;
+#pragma unroll
+        for (int d = 1; d < kC; d *= 2) {
+            const float o = __shfl_up(a, d);
+            a = lane >= d ? a + o : a;
+        }
+        const float end = __shfl(a, kC - 1);
+        const float b = lane < nt ? be : 0.0f;
+        gs[lane] = a;
+        bs[lane] = b;
+        bg[lane] = b * expf(a);
+        dec[lane] = lane < nt ? expf(end - a) : 0.0f;  // gamma_end / gamma_t
+        Gc[g + lane] = a;
     }
     __syncthreads();
-    if (tid < kC) {
-        gam[tid] = expf(gs[tid]);
-        if (tid < nt) Gc[(size_t)(t0 + tid) * H + h] = gs[tid];
-    }
 
-    // A = beta_t (gamma_t/gamma_s) K K^T, strictly lower; wave w: rows 16w..16w+15
+    // A = beta_t (gamma_t/gamma_s) K K^T, strictly lower: row block 3 - wave
     {
-        f32x4 acc[4];
+        const int tb = 3 - wave, t = 16 * tb + l16;
+        f32x4 kt[kD / 16];
 #pragma unroll
-        for (int tc = 0; tc < 4; ++tc) acc[tc] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int k0 = 0; k0 < kD; k0 += 4) {
-            const float a = Ks[(wave * 16 + l16) * KP + k0 + l4];
+        for (int kb = 0; kb < kD / 16; ++kb) kt[kb] = ld4(&Ks[t * KP + 16 * kb + 4 * l4]);
+        const float gt = gs[t], bt = bs[t];
+        for (int sb = 0; sb <= tb; ++sb) {
+            f32x4 acc[4];
 #pragma unroll
-            for (int tc = 0; tc < 4; ++tc) acc[tc] = mma(a, Ks[(tc * 16 + l16) * KP + k0 + l4], acc[tc]);
-        }
+            for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int tc = 0; tc < 4; ++tc)
+            for (int kb = 0; kb < kD / 16; ++kb) {
+                const f32x4 a = ld4(&Ks[(16 * sb + l16) * KP + 16 * kb + 4 * l4]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[j] = mma(a[j], kt[kb][j], acc[j]);
+            }
+            const f32x4 g4 = ld4(&gs[16 * sb + 4 * l4]);
+            f32x4 v;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int t = wave * 16 + l4 * 4 + i, s = tc * 16 + l16;
-                Ts[t * TP + s] = s < t ? bs[t] * expf(gs[t] - gs[s]) * acc[tc][i] : 0.0f;
+                const float p = (acc[0][i] + acc[1][i]) + (acc[2][i] + acc[3][i]);
+                v[i] = 16 * sb + 4 * l4 + i < t ? bt * expf(gt - g4[i]) * p : 0.0f;
             }
+            st4(&Ts[t * TP + 16 * sb + 4 * l4], v);
+        }
     }
 
-    // Mq[t][s] = (gamma_t/gamma_s) q_t . k_s for s <= t; wave w: rows 16w..
+    // Mq[t][s] = (gamma_t/gamma_s) q_t . k_s for s <= t: row block wave
     {
-        f32x4 m[4];
+        const float gt = gs[tq];
+        float* mq = Mq + tile * kC * kC + (size_t)wave * 4 * kBlk + lane * 4;
+        for (int sb = 0; sb <= wave; ++sb) {
+            f32x4 acc[4];
 #pragma unroll
-        for (int tc = 0; tc < 4; ++tc) m[tc] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < kD / 4; ++i) {
-            const float a = tq < nt ? qv[i] : 0.0f;
+            for (int kb = 0; kb < kD / 16; ++kb) {
+                const f32x4 a = ld4(&Ks[(16 * sb + l16) * KP + 16 * kb + 4 * l4]);
 #pragma unroll
-            for (int tc = 0; tc < 4; ++tc)
-                m[tc] = mma(a, Ks[(tc * 16 + l16) * KP + 4 * i + l4], m[tc]);
-        }
-        float* mq = Mq + ((size_t)c * H + h) * kC * kC;
-#pragma unroll
-        for (int tc = 0; tc < 4; ++tc)
+                for (int j = 0; j < 4; ++j) acc[j] = mma(a[j], qv[kb][j], acc[j]);
+            }
+            const f32x4 g4 = ld4(&gs[16 * sb + 4 * l4]);
+            f32x4 v;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int t = wave * 16 + l4 * 4 + i, s = tc * 16 + l16;
-                mq[t * kC + s] = (s <= t && t < nt) ? expf(gs[t] - gs[s]) * m[tc][i] : 0.0f;
+                const float p = (acc[0][i] + acc[1][i]) + (acc[2][i] + acc[3][i]);
+                v[i] = (16 * sb + 4 * l4 + i <= tq && tq < nt) ? expf(gt - g4[i]) * p : 0.0f;
             }
-    }
-    __syncthreads();
-
-    // T = (I + A)^-1 diag(beta) by forward substitution; lane s < 64 owns
-    // column s (T[t][s] = beta_t [t == s] - sum_{r<t} A[t][r] T[r][s]).
-    float col[kC];
-    if (tid < kC) {
-#pragma unroll
-        for (int t = 0; t < kC; ++t) {
-            float v = t == tid ? bs[t] : 0.0f;
-#pragma unroll
-            for (int r = 0; r < t; ++r) v = fmaf(-Ts[t * TP + r], col[r], v);
-            col[t] = v;
+            st4(mq + sb * kBlk, v);
         }
     }
-    __syncthreads();  // every read of A is done before T overwrites it
-    if (tid < kC) {
-#pragma unroll
-        for (int t = 0; t < kC; ++t) Ts[t * TP + tid] = col[t];
-    }
     __syncthreads();
 
-    // Wk = T diag(gamma) K and U = T V: wave w columns 32w..32w+31, all 64
-    // rows (four row tiles)
+    // inverse of the wave's diagonal block: lane l16 column l16 (the four
+    // lane groups alike), row r's value known once the rows before it have
+    // been subtracted
     {
-        f32x4 wk[4][2], u[4][2];
+        const float* A = Ts + (16 * wave) * TP + 16 * wave;
+        float* X = Xs + (16 * wave) * TP + 16 * wave + l16;
+        f32x4 ar[16][4];
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int t = 1; t < 16; ++t)
 #pragma unroll
-            for (int ct = 0; ct < 2; ++ct) {
-                wk[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-                u[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int k = 0; k < (t + 3) / 4; ++k) ar[t][k] = ld4(A + t * TP + 4 * k);
+        float x[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) x[t] = t == l16 ? 1.0f : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 15; ++r)
+#pragma unroll
+            for (int t = r + 1; t < 16; ++t) x[t] = fmaf(-ar[t][r / 4][r % 4], x[r], x[t]);
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+            if (l4 == t / 4) X[t * TP] = x[t];
+    }
+    __syncthreads();
+
+    // block (m, k) of A or X as an A operand, and of X as a B operand
+    auto rows = [&](const float* M, int m, int k) {
+        return ld4(M + (16 * m + l16) * TP + 16 * k + 4 * l4);
+    };
+    auto cols = [&](int k, int n) {
+        f32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = Xs[(16 * k + 4 * l4 + j) * TP + 16 * n + l16];
+        return v;
+    };
+    auto put = [&](int m, int n, f32x4 v) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) Xs[(16 * m + 4 * l4 + i) * TP + 16 * n + l16] = -v[i];
+    };
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (wave < 2) {  // 16 -> 32 rows
+        const int b = 2 * wave;
+        const f32x4 p = mma4(rows(Ts, b + 1, b), cols(b, b), zero);
+        put(b + 1, b, mma4(rows(Xs, b + 1, b + 1), p, zero));
+    }
+    __syncthreads();
+    {  // 32 -> 64 rows: block (m, n) of the lower left half
+        const int n = wave & 1, m = 2 + (wave >> 1);
+        f32x4 p2 = zero, p3 = zero;
+        for (int k = n; k < 2; ++k) {
+            const f32x4 x = cols(k, n);
+            p2 = mma4(rows(Ts, 2, k), x, p2);
+            p3 = mma4(rows(Ts, 3, k), x, p3);
+        }
+        f32x4 v = mma4(rows(Xs, m, 2), p2, zero);
+        if (m == 3) v = mma4(rows(Xs, 3, 3), p3, v);
+        put(m, n, v);
+    }
+    __syncthreads();
+
+    // U = X diag(beta) V, Wk = X diag(beta gamma) K (stored negated), and
+    // K^T diag(gamma_end / gamma): columns 32 wave .. + 31
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct) {
+        const int cb = 2 * wave + ct;
+        f32x4 wk[4], u[4];
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) wk[rt] = u[rt] = zero;
+#pragma unroll
+        for (int kb = 0; kb < kC / 16; ++kb) {
+            const int s = 16 * kb + 4 * l4;
+            const f32x4 b4 = ld4(&bs[s]), g4 = ld4(&bg[s]), d4 = ld4(&dec[s]);
+            f32x4 kd, kg, vb;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float kv = Ks[(s + j) * KP + 16 * cb + l16];
+                kd[j] = kv * d4[j];
+                kg[j] = kv * g4[j];
+                vb[j] = s + j < nt ? vr[kb][j][ct] * b4[j] : 0.0f;
             }
+            st4(kk + base + (size_t)(cb * 4 + kb) * kBlk + lane * 4, kd);
 #pragma unroll
-        for (int i = 0; i < kC / 4; ++i) {
-            const int s = 4 * i + l4;
-            const bool ok = s < nt;
-            const float g = gam[s];
-            const float kb0 = Ks[s * KP + 32 * wave + l16], kb1 = Ks[s * KP + 32 * wave + 16 + l16];
-            const float vb0 = ok ? vr[i][0] : 0.0f, vb1 = ok ? vr[i][1] : 0.0f;
-#pragma unroll
-            for (int rt = 0; rt < 4; ++rt) {
-                const float tv = Ts[(rt * 16 + l16) * TP + s];
-                const float tg = tv * g;
-                wk[rt][0] = mma(tg, kb0, wk[rt][0]);
-                wk[rt][1] = mma(tg, kb1, wk[rt][1]);
-                u[rt][0] = mma(tv, vb0, u[rt][0]);
-                u[rt][1] = mma(tv, vb1, u[rt][1]);
+            for (int rt = kb; rt < 4; ++rt) {
+                const f32x4 x = rows(Xs, rt, kb);
+                wk[rt] = mma4(kg, x, wk[rt]);  // transposed: rows d_k, columns t
+                u[rt] = mma4(x, vb, u[rt]);
             }
         }
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int t = rt * 16 + l4 * 4 + i;
-                    if (t < nt) {
-                        const size_t o = rix(t0 + t, h, H) + 32 * wave + 16 * ct + l16;
-                        Wk[o] = wk[rt][ct][i];
-                        U[o] = u[rt][ct][i];
-                    }
-                }
+        for (int rt = 0; rt < 4; ++rt) {
+            const size_t o = base + (size_t)(rt * 8 + cb) * kBlk + lane * 4;
+            st4(Wk + o, -wk[rt]);
+            st4(U + o, u[rt]);
+        }
     }
 }
 
-// Per (head, 16 value columns), chunks in order, with two roles a SIMD:
-// waves 0-3 run the state chain of chunk c,
-//   W = U - Wk S,  S = gamma_end S + K^T diag(gamma_end / gamma) W,
-// the only products that depend on the state (wave w: W rows 16w.., state
-// rows 32w..); waves 4-7 meanwhile form the outputs of chunk c-1,
-//   O = (gamma_t (Q S) + Mq W) / sqrt(d),
-// Q S beside the chain's W and Mq W beside its state update, from the state
-// and W that chunk left in LDS, so that work fills the chain's waits instead
-// of lengthening it. The output waves also stage each chunk's k rows in LDS
-// (whole rows, 16-byte loads) for the state update. The state is kept in
-// three LDS slots (S_c read by the chain, S_{c+1} written, S_{c-1} read by
-// the output waves), W and the cumulative gates in two. The chunk operands
-// do not depend on the state: each is loaded for the next chunk right after
-// its last use in this one, from buffers padded to whole chunks (rows past T
-// are never used: every operand from them is replaced by zero with a
-// select). Every product runs its K index as 16 kb + 4 l4 + j on lane
-// (l16, l4), so the LDS operand of four consecutive products is one 16-byte
-// read: the state and W slices are stored transposed ([16][K + 4]).
-constexpr int KT = kD + 4;  // pitch of a transposed state slice
-constexpr int TT = kC + 4;  // pitch of a transposed W slice
+// Per (head, 16 value columns), chunks in order:
+//   W = U - Wk S,  S = gamma_end S + K^T diag(gamma_end / gamma) W.
+// Only these two products depend on the state; the state before each chunk
+// and W (over U) are written out for the outputs. A serial chain, bound by
+// the matrix cores' time of its 64 products a SIMD and chunk and by the two
+// exchanges through LDS: wave w takes row block w % 4 of W over half of K
+// (w / 4; the halves meet as W is read), then row block w of the state. All
+// operands arrive in operand order, kRing chunks ahead.
+constexpr int kRing = 3;
 
-__global__ __launch_bounds__(512) void k_dn_chunk_inter(
-    const float* __restrict__ qn, const float* __restrict__ kn, const float* __restrict__ U,
-    const float* __restrict__ Wk, const float* __restrict__ Mq, const float* __restrict__ Gc,
-    int T, int H, float* __restrict__ state, float* __restrict__ O) {
-    __shared__ __attribute__((aligned(16))) float St[3][CB * KT];
-    __shared__ __attribute__((aligned(16))) float Wt[2][CB * TT];
-    __shared__ __attribute__((aligned(16))) float gs[2][kC];
-    __shared__ __attribute__((aligned(16))) float dec[kC];
-    __shared__ __attribute__((aligned(16))) float Ks[kC * KP];
-    const int h = blockIdx.x, jb = blockIdx.y * CB;
+__global__ __launch_bounds__(512) void k_dn_chunk_chain(
+    const float* __restrict__ Kt, const float* __restrict__ Wk, float* UW,
+    const float* __restrict__ Gc, int T, int H, float* __restrict__ state,
+    float* __restrict__ Sall) {
+    __shared__ __attribute__((aligned(16))) float Ss[8 * kBlk];
+    __shared__ __attribute__((aligned(16))) float Wp[2][4 * kBlk];
+    const int h = blockIdx.x, jt = blockIdx.y, jb = jt * CB;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: the roles branch on it
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, l4 = lane >> 4;
-    const int w4 = wave & 3;
+    const int rt = wave & 3, kh = wave >> 2;
     const int nch = (T + kC - 1) / kC;
-    const size_t RS = (size_t)H * kD;  // a row of every head
-    const size_t CS = kC * RS;         // a chunk of rows
-    const int tr = w4 * 16 + l16;      // A-operand row of this wave's tiles
-    auto lds4 = [](const float* p) { return *reinterpret_cast<const float4*>(p); };
-    auto sto4 = [](float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; };
+    const size_t CS = (size_t)H * kC * kD;  // a chunk of every head
+    const size_t at = (size_t)h * kC * kD + lane * 4;
+    const float* wk_p = Wk + at + (rt * 8 + 4 * kh) * kBlk;
+    const float* kt_p = Kt + at + wave * 4 * kBlk;
+    float* uw_p = UW + at + (rt * 8 + jt) * kBlk;
+    float* s_p = Sall + 2 * (size_t)h * kC * kD + (jt * 8 + wave) * kBlk + lane * 4;
+    const float* g_p = Gc + (size_t)h * kC + kC - 1;
 
-    // Each role runs its own loop (so each loop's load waits count only its
-    // own loads); both meet two barriers a pass, nch + 1 passes.
-    if (wave < 4) {
-        // state rows 32w .. 32w+31 (two 16-row tiles), columns jb .. jb+15
-        float* Sg = state + (size_t)h * kD * kD;
-        f32x4 sacc[2];
-        float4 pw[8];
-        float pu[4], pg = 0.0f, pge = 0.0f;
-        const float* wk_b = Wk + tr * RS + h * kD + 4 * l4;
-        const float* u_b = U + (w4 * 16 + l4 * 4) * RS + h * kD + jb + l16;
-        auto load_g = [&](int c) {
-            pg = Gc[((size_t)c * kC + lane) * H + h];  // row lane of the chunk (wave 0 uses it)
-            pge = Gc[((size_t)c * kC + min(kC, T - c * kC) - 1) * H + h];
-        };
-        auto load_wu = [&](int c) {
-            const size_t cs = (size_t)c * CS;
+    f32x4 wk[kRing][4], kt[kRing][4], u[kRing];
+    float ge[kRing];
+    auto load_w = [&](int s, int c) {
 #pragma unroll
-            for (int kb = 0; kb < 8; ++kb) pw[kb] = *reinterpret_cast<const float4*>(wk_b + cs + 16 * kb);
+        for (int kb = 0; kb < 4; ++kb) wk[s][kb] = ld4(wk_p + (size_t)c * CS + kb * kBlk);
+        if (kh == 0) u[s] = ld4(uw_p + (size_t)c * CS);
+    };
+    auto load_k = [&](int s, int c) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) pu[i] = u_b[cs + i * RS];
-        };
+        for (int kb = 0; kb < 4; ++kb) kt[s][kb] = ld4(kt_p + (size_t)c * CS + kb * kBlk);
+        ge[s] = g_p[(size_t)c * H * kC];
+    };
+    float* Sg = state + (size_t)h * kD * kD + (size_t)(16 * wave + 4 * l4) * kD + jb + l16;
+    f32x4 sacc;  // state rows 16 wave + 4 l4 + i, column jb + l16
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const int r0 = (2 * w4 + tt) * 16 + l4 * 4;
+    for (int i = 0; i < 4; ++i) sacc[i] = Sg[i * kD];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sacc[tt][i] = Sg[(size_t)(r0 + i) * kD + jb + l16];
-            sto4(&St[0][l16 * KT + r0], sacc[tt]);
-        }
-        load_g(0);
-        load_wu(0);
-        // Every load of the preamble lands before the loop: the wait counts
-        // inside it then follow the loop's own load order (entered with the
-        // preamble's loads pending, in another order, they wait for all).
-        landed(pg);
-        landed(pge);
+    for (int s = 0; s < kRing; ++s) {
+        u[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+        load_w(s, min(s, nch - 1));
+        load_k(s, min(s, nch - 1));
+    }
+    st4(&Ss[wave * kBlk + lane * 4], sacc);
+    __syncthreads();
+    const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c0 = 0; c0 < nch; c0 += kRing) {
 #pragma unroll
-        for (int kb = 0; kb < 8; ++kb) landed(pw[kb]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) landed(pu[i]);
-        __syncthreads();
-        for (int c = 0; c < nch; ++c) {
-            const int cn = min(c + 1, nch - 1);
-            const int nt = min(kC, T - c * kC);
-            const bool tv = tr < nt;
-            const float* Sc = St[c % 3] + l16 * KT + 4 * l4;
-            if (wave == 0) {
-                gs[c & 1][lane] = lane < nt ? pg : 0.0f;
-                dec[lane] = lane < nt ? expf(pge - pg) : 0.0f;  // gamma_end / gamma_t
-            }
-            const float ge = expf(pge);
-            load_g(cn);
-            // W = U - Wk S (four independent chains: a chain of dependent
-            // products waits out each one's latency)
-            f32x4 wc[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) wc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kb = 0; kb < 8; ++kb) {
-                const float a[4] = {pw[kb].x, pw[kb].y, pw[kb].z, pw[kb].w};
-                const float4 b4 = lds4(Sc + 16 * kb);
-                const float b[4] = {b4.x, b4.y, b4.z, b4.w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) wc[j] = mma(tv ? a[j] : 0.0f, b[j], wc[j]);
-            }
-            f32x4 wv;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = w4 * 16 + l4 * 4 + i;
-                wv[i] = t < nt ? pu[i] - ((wc[0][i] + wc[1][i]) + (wc[2][i] + wc[3][i])) : 0.0f;
-            }
-            sto4(&Wt[c & 1][l16 * TT + w4 * 16 + l4 * 4], wv);
-            load_wu(cn);
-            __syncthreads();  // W of chunk c and its gates are in LDS
-            // S = gamma_end S + K^T diag(gamma_end / gamma) W
-            const float* Wc = Wt[c & 1] + l16 * TT + 4 * l4;
-            const float* Kc = Ks + 4 * l4 * KP + 2 * w4 * 16 + l16;
-            f32x4 du[2][2];
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) du[tt][0] = du[tt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < kRing; ++s) {
+            const int c = c0 + s;
+            if (c >= nch) break;
+            const int cn = min(c + kRing, nch - 1);
+            f32x4 w0 = u[s], w1 = zero;
 #pragma unroll
             for (int kb = 0; kb < 4; ++kb) {
-                const float4 w4v = lds4(Wc + 16 * kb);
-                const float4 d4 = lds4(&dec[16 * kb + 4 * l4]);
-                const float b[4] = {w4v.x * d4.x, w4v.y * d4.y, w4v.z * d4.z, w4v.w * d4.w};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const bool ok = 16 * kb + 4 * l4 + j < nt;
-#pragma unroll
-                    for (int tt = 0; tt < 2; ++tt) {
-                        const float kv = Kc[(16 * kb + j) * KP + 16 * tt];
-                        du[tt][j & 1] = mma(ok ? kv : 0.0f, b[j], du[tt][j & 1]);
-                    }
-                }
+                const f32x4 b = ld4(&Ss[(4 * kh + kb) * kBlk + lane * 4]);
+                w0 = mma(wk[s][kb][0], b[0], w0);
+                w1 = mma(wk[s][kb][1], b[1], w1);
+                w0 = mma(wk[s][kb][2], b[2], w0);
+                w1 = mma(wk[s][kb][3], b[3], w1);
             }
-            float* Sn = St[(c + 1) % 3];
+            st4(&Wp[kh][rt * kBlk + lane * 4], w0 + w1);
+            st4(s_p + (size_t)c * 2 * CS, sacc);
+            load_w(s, cn);
+            __syncthreads();  // W of chunk c is in LDS, its state was read
+            f32x4 d0 = sacc * expf(ge[s]), d1 = zero;
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    sacc[tt][i] = sacc[tt][i] * ge + (du[tt][0][i] + du[tt][1][i]);
-                sto4(&Sn[l16 * KT + (2 * w4 + tt) * 16 + l4 * 4], sacc[tt]);
+            for (int kb = 0; kb < 4; ++kb) {
+                const f32x4 b = ld4(&Wp[0][kb * kBlk + lane * 4]) + ld4(&Wp[1][kb * kBlk + lane * 4]);
+                if (wave == kb) st4(uw_p + (size_t)c * CS, b);
+                d0 = mma(kt[s][kb][0], b[0], d0);
+                d1 = mma(kt[s][kb][1], b[1], d1);
+                d0 = mma(kt[s][kb][2], b[2], d0);
+                d1 = mma(kt[s][kb][3], b[3], d1);
             }
-            __syncthreads();  // S of chunk c+1 is in LDS; this pass's slot reads are done
-        }
-        __syncthreads();  // the output waves' last pass
-        __syncthreads();
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                Sg[(size_t)((2 * w4 + tt) * 16 + l4 * 4 + i) * kD + jb + l16] = sacc[tt][i];
-    } else {
-        // outputs of the chunk before: q and Mq rows 16w'.. of it
-        const float rsd = 1.0f / sqrtf((float)kD);
-        const size_t MS = (size_t)H * kC * kC;
-        float4 pq[8], pm[4];
-        const float* q_b = qn + tr * RS + h * kD + 4 * l4;
-        const float* m_b = Mq + ((size_t)h * kC + tr) * kC + 4 * l4;
-        auto load_out = [&](int c) {
-#pragma unroll
-            for (int kb = 0; kb < 8; ++kb)
-                pq[kb] = *reinterpret_cast<const float4*>(q_b + (size_t)c * CS + 16 * kb);
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb)
-                pm[kb] = *reinterpret_cast<const float4*>(m_b + (size_t)c * MS + 16 * kb);
-        };
-        // k rows of a chunk: thread o = tid - 256 moves float4 o + 256 i
-        float4 pkk[8];
-        const int o = tid - 256;
-        auto load_kk = [&](int c) {
-            const float* base = kn + (size_t)c * CS + h * kD;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int e = o + 256 * i;
-                pkk[i] = *reinterpret_cast<const float4*>(base + (e >> 5) * RS + (e & 31) * 4);
-            }
-        };
-        auto store_kk = [&]() {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int e = o + 256 * i;
-                *reinterpret_cast<float4*>(&Ks[(e >> 5) * KP + (e & 31) * 4]) = pkk[i];
-            }
-        };
-        load_out(0);
-        load_kk(0);
-        store_kk();
-        if (nch > 1) load_kk(1);
-#pragma unroll
-        for (int kb = 0; kb < 8; ++kb) landed(pq[kb]);
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) landed(pm[kb]);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) landed(pkk[i]);
-        __syncthreads();
-        for (int c = 0; c <= nch; ++c) {
-            const int cp = c - 1;
-            const int nt = min(kC, T - cp * kC);
-            const bool tv = tr < nt;
-            f32x4 qc[4];
-            if (c > 0 && c < nch) {  // k rows of chunk c for its state update
-                store_kk();
-                if (c + 1 < nch) load_kk(c + 1);
-            }
-            if (c > 0) {  // Q S, beside the chain's W = U - Wk S
-                const float* Sp = St[cp % 3] + l16 * KT + 4 * l4;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) qc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int kb = 0; kb < 8; ++kb) {
-                    const float a[4] = {pq[kb].x, pq[kb].y, pq[kb].z, pq[kb].w};
-                    const float4 b4 = lds4(Sp + 16 * kb);
-                    const float b[4] = {b4.x, b4.y, b4.z, b4.w};
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) qc[j] = mma(tv ? a[j] : 0.0f, b[j], qc[j]);
-                }
-            }
-            __syncthreads();
-            if (c > 0) {  // Mq W and the outputs, beside the chain's state update
-                const float* Wp = Wt[cp & 1] + l16 * TT + 4 * l4;
-                f32x4 mc[2];
-                mc[0] = mc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int kb = 0; kb < 4; ++kb) {
-                    const float a[4] = {pm[kb].x, pm[kb].y, pm[kb].z, pm[kb].w};
-                    const float4 b4 = lds4(Wp + 16 * kb);
-                    const float b[4] = {b4.x, b4.y, b4.z, b4.w};
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) mc[j & 1] = mma(tv ? a[j] : 0.0f, b[j], mc[j & 1]);
-                }
-                if (c < nch) load_out(c);
-                const float4 g4 = lds4(&gs[cp & 1][w4 * 16 + l4 * 4]);
-                const float g[4] = {g4.x, g4.y, g4.z, g4.w};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int t = w4 * 16 + l4 * 4 + i;
-                    if (t < nt)
-                        O[((size_t)cp * kC + t) * RS + h * kD + jb + l16] =
-                            (expf(g[i]) * ((qc[0][i] + qc[2][i]) + (qc[1][i] + qc[3][i])) +
-                             (mc[0][i] + mc[1][i])) * rsd;
-                }
-            }
-            __syncthreads();
+            load_k(s, cn);
+            sacc = d0 + d1;
+            st4(&Ss[wave * kBlk + lane * 4], sacc);
+            __syncthreads();  // the state of chunk c + 1 is in LDS, W was read
         }
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) Sg[i * kD] = sacc[i];
 }
 
-// Per (16 rows, head): a wave a row at a time (its two 64-column halves
-// summed as the decode step's two waves are), and the conv ring rows of the
-// last three positions.
-__global__ __launch_bounds__(256) void k_dn_chunk_post(
-    const float* __restrict__ O, const float* __restrict__ proj, int ldp, int T,
-    const float* __restrict__ norm_w, float* __restrict__ out, int ldo, int H,
+// Per (chunk, head), transposed (rows value columns, columns t):
+//   O = (gamma_t (Q S) + Mq W) / sqrt(d),
+// wave w value columns 32 w .. + 31 of all 64 rows; then the head RMSNorm
+// (the waves' sums of squares meet in LDS) and the SiLU(z) gate, and the conv
+// ring rows of the last three positions. V4: proj and out rows take 16-byte
+// accesses.
+template <bool V4>
+__global__ __launch_bounds__(256, 2) void k_dn_chunk_out(
+    const float* __restrict__ qn, const float* __restrict__ Sall, const float* __restrict__ Mq,
+    const float* __restrict__ W, const float* __restrict__ Gc, const float* __restrict__ proj,
+    int ldp, int T, const float* __restrict__ norm_w, float* __restrict__ out, int ldo, int H,
     float* __restrict__ conv_state, int p0) {
-    const int t0 = blockIdx.x * kPR, h = blockIdx.y;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nt = min(kPR, T - t0);
+    __shared__ float red[4][kC];
+    const int c = blockIdx.x, h = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, l4 = lane >> 4;
+    const int t0 = c * kC, nt = min(kC, T - t0);
     const int HD = H * kD, C = 3 * HD;
-    const float nw0 = norm_w[lane], nw1 = norm_w[lane + 64];
-    for (int r = wave; r < nt; r += 4) {
-        const int t = t0 + r;
-        const float* pr = proj + (size_t)t * ldp;
-        const float o0 = O[rix(t, h, H) + lane], o1 = O[rix(t, h, H) + lane + 64];
-        const float z0 = pr[3 * HD + h * kD + lane], z1 = pr[3 * HD + h * kD + lane + 64];
-        const float tot = wave_sum(o0 * o0) + wave_sum(o1 * o1);
+    const size_t tile = (size_t)c * H + h;
+    const size_t base = tile * kC * kD;
+    const int col = h * kD + 32 * wave + 4 * l4;  // + 16 d + i
+    auto load = [&](const float* p) {
+        if constexpr (V4) return ld4(p);
+        else return f32x4{p[0], p[1], p[2], p[3]};
+    };
+    f32x4 z[2][4];
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+        const float* zr = proj + (size_t)(t0 + min(16 * tb + l16, nt - 1)) * ldp + 3 * HD + col;
+#pragma unroll
+        for (int d = 0; d < 2; ++d) z[d][tb] = load(zr + 16 * d);
+    }
+    f32x4 nw[2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) nw[d][i] = norm_w[32 * wave + 16 * d + 4 * l4 + i];
+    float g[4];
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) g[tb] = Gc[tile * kC + 16 * tb + l16];
+
+    f32x4 o[2][4];
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) o[d][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // rows past the chunk's last feed only their own columns, never stored
+    const float* s_p = Sall + 2 * base + (size_t)wave * 16 * kBlk + lane * 4;
+    const float* q_p = qn + base + (size_t)l16 * kD + 4 * l4;
+#pragma unroll
+    for (int kb = 0; kb < kD / 16; ++kb) {
+        f32x4 sv[2], qv[4];
+#pragma unroll
+        for (int d = 0; d < 2; ++d) sv[d] = ld4(s_p + (d * 8 + kb) * kBlk);
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) qv[tb] = ld4(q_p + 16 * tb * kD + 16 * kb);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) o[d][tb] = mma(sv[d][j], qv[tb][j], o[d][tb]);
+    }
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+        const float gt = expf(g[tb]);
+#pragma unroll
+        for (int d = 0; d < 2; ++d) o[d][tb] *= gt;
+    }
+    const float* w_p = W + base + (size_t)2 * wave * kBlk + lane * 4;
+    const float* m_p = Mq + tile * kC * kC + lane * 4;
+#pragma unroll
+    for (int kb = 0; kb < kC / 16; ++kb) {
+        f32x4 wv[2], mv[4];
+#pragma unroll
+        for (int d = 0; d < 2; ++d) wv[d] = ld4(w_p + (kb * 8 + d) * kBlk);
+#pragma unroll
+        for (int tb = kb; tb < 4; ++tb) mv[tb] = ld4(m_p + (tb * 4 + kb) * kBlk);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int tb = kb; tb < 4; ++tb) o[d][tb] = mma(wv[d][j], mv[tb][j], o[d][tb]);
+    }
+    const float rsd = 1.0f / sqrtf((float)kD);
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            o[d][tb] *= rsd;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ss = fmaf(o[d][tb][i], o[d][tb][i], ss);
+        }
+        ss = xor32_add(xor16_add(ss));
+        if (l4 == 0) red[wave][16 * tb + l16] = ss;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+        const int t = 16 * tb + l16;
+        const float tot = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
         const float sn = 1.0f / sqrtf(tot / (float)kD + 1e-6f);
-        out[(size_t)t * ldo + h * kD + lane] = ((o0 * sn) * nw0) * silu_f(z0);
-        out[(size_t)t * ldo + h * kD + lane + 64] = ((o1 * sn) * nw1) * silu_f(z1);
-        if (t >= T - 3) {  // ring row of position p0 + t keeps its conv input
-            const int row = (p0 + t) % 3;
-            for (int i = lane; i < 3 * kD; i += 64) {
-                const int ch = (i / kD) * HD + h * kD + i % kD;
-                conv_state[(size_t)row * C + ch] = pr[ch];
+        if (t < nt) {
+            float* dst = out + (size_t)(t0 + t) * ldo + col;
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                f32x4 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = ((o[d][tb][i] * sn) * nw[d][i]) * silu_f(z[d][tb][i]);
+                if constexpr (V4) {
+                    st4(dst + 16 * d, v);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) dst[16 * d + i] = v[i];
+                }
             }
+        }
+    }
+    for (int t = max(t0, T - 3); t < t0 + nt; ++t) {  // ring row of position p0 + t: its conv input
+        const int row = (p0 + t) % 3;
+        for (int i = tid; i < 3 * kD; i += 256) {
+            const int ch = (i / kD) * HD + h * kD + i % kD;
+            conv_state[(size_t)row * C + ch] = proj[(size_t)t * ldp + ch];
         }
     }
 }
 
 size_t a256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// kn becomes the decayed K^T, U the chunks' W; the states before each chunk
+// (two rows' worth) take v's place, which only the intra kernel reads, and
+// the rows after it.
 struct ChunkWork {
-    float *qn, *kn, *vv, *U, *Wk, *O, *alpha, *beta, *Gc, *Mq;
+    float *qn, *kn, *U, *Wk, *vv, *alpha, *beta, *Gc, *Mq;
     size_t bytes;
 };
 
 ChunkWork carve(void* base, int T, int H) {
     ChunkWork w{};
-    // rows and gates padded to whole chunks: the state chain reads a whole
-    // chunk's operands and masks the rows past T
-    const int nch = (T + kC - 1) / kC;
+    const int nch = (T + kC - 1) / kC;  // whole chunks
     const size_t rows = a256((size_t)nch * kC * H * kD * sizeof(float));
     const size_t sc = a256((size_t)nch * kC * H * sizeof(float));
+    const size_t mq = a256((size_t)nch * H * kC * kC * sizeof(float));
     char* p = reinterpret_cast<char*>(base);
     auto take = [&](size_t b) {
         float* r = reinterpret_cast<float*>(p);
@@ -597,15 +614,14 @@ ChunkWork carve(void* base, int T, int H) {
     };
     w.qn = take(rows);
     w.kn = take(rows);
-    w.vv = take(rows);
     w.U = take(rows);
     w.Wk = take(rows);
-    w.O = take(rows);
+    w.vv = take(2 * rows);
     w.alpha = take(sc);
     w.beta = take(sc);
     w.Gc = take(sc);
-    w.Mq = take(a256((size_t)nch * H * kC * kC * sizeof(float)));
-    w.bytes = 6 * rows + 3 * sc + a256((size_t)nch * H * kC * kC * sizeof(float));
+    w.Mq = take(mq);
+    w.bytes = 6 * rows + 3 * sc + mq;
     return w;
 }
 
@@ -640,12 +656,15 @@ extern "C" int qlm_deltanet_prefill_chunked(const float* proj, int ldp, int T, f
                        w.alpha, w.beta, T, H, w.U, w.Wk, w.Mq, w.Gc);
     rc = qlm_launch_status();
     if (rc != QLM_OK) return rc;
-    hipLaunchKernelGGL(k_dn_chunk_inter, dim3(H, kD / CB), dim3(512), 0, st, w.qn, w.kn, w.U,
-                       w.Wk, w.Mq, w.Gc, T, H, state, w.O);
+    hipLaunchKernelGGL(k_dn_chunk_chain, dim3(H, kD / CB), dim3(512), 0, st, w.kn, w.Wk, w.U, w.Gc,
+                       T, H, state, w.vv);
     rc = qlm_launch_status();
     if (rc != QLM_OK) return rc;
-    hipLaunchKernelGGL(k_dn_chunk_post, dim3(nrb, H), dim3(256), 0, st, w.O, proj, ldp, T, norm_w,
-                       out, ldo, H, conv_state, p0);
+    const bool v4 = ldp % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)proj & 15u) == 0 &&
+                    ((uintptr_t)out & 15u) == 0;
+    hipLaunchKernelGGL(v4 ? k_dn_chunk_out<true> : k_dn_chunk_out<false>, dim3(nch, H), dim3(256), 0,
+                       st, w.qn, w.vv, w.Mq, w.U, w.Gc, proj, ldp, T, norm_w, out, ldo, H,
+                       conv_state, p0);
     return qlm_launch_status();
 }
 

@@ -752,6 +752,47 @@ def test_deltanet_prefill_chunked(hip, orc, rng, p0, T):
         assert rel_err(out, ref) < 1e-4
 
 
+@pytest.mark.parametrize("H,T,pad,same", [(1, 16, 0, False), (3, 17, 1, False), (5, 33, 2, False),
+                                          (2, 63, 3, False), (3, 129, 1, False),
+                                          (8, 193, 4, False), (9, 255, 0, False),
+                                          (2, 320, 0, True)])
+def test_deltanet_prefill_chunked_edges(hip, rng, H, T, pad, same):
+    """Edges of the blocks of 16 rows and of the chunk ring, head counts off
+    the multiples of 8, row strides without 16-byte alignment, and a prompt of
+    one repeated row with almost no decay (every k . k is 1: the triangular
+    systems are as full as they get). 1e-4 of the row-by-row recurrence, as
+    the entry point states."""
+    d, p0 = 128, 4
+    HD = H * d
+    ldp, ldo = 4 * HD + 2 * H + pad, HD + pad
+    wt = (rng.standard_normal((4, 3 * HD)) * 0.3).astype(np.float32)
+    A_log = np.log(rng.uniform(1, 16, H)).astype(np.float32)
+    dtb = (rng.standard_normal(H) * 0.5 - (12 if same else 4)).astype(np.float32)
+    nw = (1 + rng.standard_normal(d) * 0.02).astype(np.float32)
+    conv = (rng.standard_normal((3, 3 * HD)) * 0.5).astype(np.float32)
+    S = (rng.standard_normal((H, d, d)) * 0.05).astype(np.float32)
+    proj = (rng.standard_normal((1 if same else T, ldp)) * 0.6).astype(np.float32)
+    proj = np.ascontiguousarray(np.broadcast_to(proj, (T, ldp)))
+    args = [dev(hip, a) for a in (wt, A_log, dtb, nw)]
+    dproj = dev(hip, proj)
+    nbytes = hip.lib().qlm_deltanet_chunk_workspace_bytes(T, H, d)
+    work = hip.DeviceBuffer(nbytes)
+    got = []
+    for chunked in (False, True):
+        dconv, dS, do = dev(hip, conv), dev(hip, S), dev(hip, np.full((T, ldo), 7, np.float32))
+        say("deltanet_prefill edges", H, T, pad, same, chunked)
+        name = "qlm_deltanet_prefill" + ("_chunked" if chunked else "")
+        tail = [work, nbytes, None] if chunked else [None]
+        hip.call(name, dproj, ldp, T, dconv, *args, dS, p0, do, ldo, H, d, *tail)
+        got.append((do.to_numpy((T, ldo), np.float32), dS.to_numpy(S.shape, np.float32),
+                    dconv.to_numpy(conv.shape, np.float32)))
+    (o1, S1, c1), (o2, S2, c2) = got
+    assert rel_err(o2[:, :HD], o1[:, :HD]) < 1e-4
+    assert np.all(o2[:, HD:] == 7)
+    assert rel_err(S2, S1) < 1e-4
+    assert np.array_equal(c2, c1)
+
+
 @pytest.mark.parametrize("n_q,n_kv,hd,rot,gated,p0,T", [(16, 4, 128, 32, 1, 0, 300),
                                                         (16, 4, 128, 32, 1, 37, 90),
                                                         (16, 2, 256, 64, 0, 10, 40),
