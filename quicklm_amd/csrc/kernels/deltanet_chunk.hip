@@ -464,20 +464,23 @@ __global__ __launch_bounds__(512) void k_dn_chunk_chain(
 //   O = (gamma_t (Q S) + Mq W) / sqrt(d),
 // wave w value columns 32 w .. + 31 of all 64 rows; then the head RMSNorm
 // (the waves' sums of squares meet in LDS) and the SiLU(z) gate, and the conv
-// ring rows of the last three positions. V4: proj and out rows take 16-byte
-// accesses.
-template <bool V4>
+// ring rows of the last three positions. A workgroup takes NB row blocks: all
+// four, or one where the chunks are too few to fill the chip (66 rows, 16
+// heads: 15.2 -> 7.2 us). V4: proj and out rows take 16-byte accesses.
+template <int NB, bool V4>
 __global__ __launch_bounds__(256, 2) void k_dn_chunk_out(
     const float* __restrict__ qn, const float* __restrict__ Sall, const float* __restrict__ Mq,
     const float* __restrict__ W, const float* __restrict__ Gc, const float* __restrict__ proj,
     int ldp, int T, const float* __restrict__ norm_w, float* __restrict__ out, int ldo, int H,
     float* __restrict__ conv_state, int p0) {
-    __shared__ float red[4][kC];
-    const int c = blockIdx.x, h = blockIdx.y;
+    __shared__ float red[4][16 * NB];
+    const int c = blockIdx.x / (4 / NB), h = blockIdx.y;
+    const int rb = blockIdx.x % (4 / NB) * NB;  // first row block
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, l4 = lane >> 4;
     const int t0 = c * kC, nt = min(kC, T - t0);
+    if (16 * rb >= nt) return;
     const int HD = H * kD, C = 3 * HD;
     const size_t tile = (size_t)c * H + h;
     const size_t base = tile * kC * kD;
@@ -486,10 +489,10 @@ __global__ __launch_bounds__(256, 2) void k_dn_chunk_out(
         if constexpr (V4) return ld4(p);
         else return f32x4{p[0], p[1], p[2], p[3]};
     };
-    f32x4 z[2][4];
+    f32x4 z[2][NB];
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
-        const float* zr = proj + (size_t)(t0 + min(16 * tb + l16, nt - 1)) * ldp + 3 * HD + col;
+    for (int tb = 0; tb < NB; ++tb) {
+        const float* zr = proj + (size_t)(t0 + min(16 * (rb + tb) + l16, nt - 1)) * ldp + 3 * HD + col;
 #pragma unroll
         for (int d = 0; d < 2; ++d) z[d][tb] = load(zr + 16 * d);
     }
@@ -498,34 +501,45 @@ __global__ __launch_bounds__(256, 2) void k_dn_chunk_out(
     for (int d = 0; d < 2; ++d)
 #pragma unroll
         for (int i = 0; i < 4; ++i) nw[d][i] = norm_w[32 * wave + 16 * d + 4 * l4 + i];
-    float g[4];
+    float g[NB];
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) g[tb] = Gc[tile * kC + 16 * tb + l16];
+    for (int tb = 0; tb < NB; ++tb) g[tb] = Gc[tile * kC + 16 * (rb + tb) + l16];
 
-    f32x4 o[2][4];
+    f32x4 o[2][NB];
 #pragma unroll
     for (int d = 0; d < 2; ++d)
 #pragma unroll
-        for (int tb = 0; tb < 4; ++tb) o[d][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int tb = 0; tb < NB; ++tb) o[d][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
     // rows past the chunk's last feed only their own columns, never stored
     const float* s_p = Sall + 2 * base + (size_t)wave * 16 * kBlk + lane * 4;
-    const float* q_p = qn + base + (size_t)l16 * kD + 4 * l4;
+    const float* q_p = qn + base + (size_t)(16 * rb + l16) * kD + 4 * l4;
+    // one row block: every operand is requested before the first product
+    constexpr int PF = NB == 1 ? kD / 16 : 1;
+    f32x4 sv[PF][2], qv[PF][NB];
+    auto load_sq = [&](int kb) {
+#pragma unroll
+        for (int d = 0; d < 2; ++d) sv[kb % PF][d] = ld4(s_p + (d * 8 + kb) * kBlk);
+#pragma unroll
+        for (int tb = 0; tb < NB; ++tb) qv[kb % PF][tb] = ld4(q_p + 16 * tb * kD + 16 * kb);
+    };
+    if constexpr (PF > 1) {
+#pragma unroll
+        for (int kb = 0; kb < PF; ++kb) load_sq(kb);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int kb = 0; kb < kD / 16; ++kb) {
-        f32x4 sv[2], qv[4];
-#pragma unroll
-        for (int d = 0; d < 2; ++d) sv[d] = ld4(s_p + (d * 8 + kb) * kBlk);
-#pragma unroll
-        for (int tb = 0; tb < 4; ++tb) qv[tb] = ld4(q_p + 16 * tb * kD + 16 * kb);
+        if constexpr (PF == 1) load_sq(kb);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int d = 0; d < 2; ++d)
 #pragma unroll
-                for (int tb = 0; tb < 4; ++tb) o[d][tb] = mma(sv[d][j], qv[tb][j], o[d][tb]);
+                for (int tb = 0; tb < NB; ++tb)
+                    o[d][tb] = mma(sv[kb % PF][d][j], qv[kb % PF][tb][j], o[d][tb]);
     }
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
+    for (int tb = 0; tb < NB; ++tb) {
         const float gt = expf(g[tb]);
 #pragma unroll
         for (int d = 0; d < 2; ++d) o[d][tb] *= gt;
@@ -534,21 +548,22 @@ __global__ __launch_bounds__(256, 2) void k_dn_chunk_out(
     const float* m_p = Mq + tile * kC * kC + lane * 4;
 #pragma unroll
     for (int kb = 0; kb < kC / 16; ++kb) {
-        f32x4 wv[2], mv[4];
+        if (NB < 4 && kb >= rb + NB) break;
+        f32x4 wv[2], mv[NB];
 #pragma unroll
         for (int d = 0; d < 2; ++d) wv[d] = ld4(w_p + (kb * 8 + d) * kBlk);
 #pragma unroll
-        for (int tb = kb; tb < 4; ++tb) mv[tb] = ld4(m_p + (tb * 4 + kb) * kBlk);
+        for (int tb = NB < 4 ? 0 : kb; tb < NB; ++tb) mv[tb] = ld4(m_p + ((rb + tb) * 4 + kb) * kBlk);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int d = 0; d < 2; ++d)
 #pragma unroll
-                for (int tb = kb; tb < 4; ++tb) o[d][tb] = mma(wv[d][j], mv[tb][j], o[d][tb]);
+                for (int tb = NB < 4 ? 0 : kb; tb < NB; ++tb) o[d][tb] = mma(wv[d][j], mv[tb][j], o[d][tb]);
     }
     const float rsd = 1.0f / sqrtf((float)kD);
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
+    for (int tb = 0; tb < NB; ++tb) {
         float ss = 0.0f;
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
@@ -561,9 +576,9 @@ __global__ __launch_bounds__(256, 2) void k_dn_chunk_out(
     }
     __syncthreads();
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
-        const int t = 16 * tb + l16;
-        const float tot = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+    for (int tb = 0; tb < NB; ++tb) {
+        const int tr = 16 * tb + l16, t = 16 * rb + tr;
+        const float tot = (red[0][tr] + red[1][tr]) + (red[2][tr] + red[3][tr]);
         const float sn = 1.0f / sqrtf(tot / (float)kD + 1e-6f);
         if (t < nt) {
             float* dst = out + (size_t)(t0 + t) * ldo + col;
@@ -581,7 +596,8 @@ __global__ __launch_bounds__(256, 2) void k_dn_chunk_out(
             }
         }
     }
-    for (int t = max(t0, T - 3); t < t0 + nt; ++t) {  // ring row of position p0 + t: its conv input
+    // ring row of position p0 + t: its conv input
+    for (int t = max(t0 + 16 * rb, T - 3); t < t0 + min(16 * (rb + NB), nt); ++t) {
         const int row = (p0 + t) % 3;
         for (int i = tid; i < 3 * kD; i += 256) {
             const int ch = (i / kD) * HD + h * kD + i % kD;
@@ -662,9 +678,14 @@ extern "C" int qlm_deltanet_prefill_chunked(const float* proj, int ldp, int T, f
     if (rc != QLM_OK) return rc;
     const bool v4 = ldp % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)proj & 15u) == 0 &&
                     ((uintptr_t)out & 15u) == 0;
-    hipLaunchKernelGGL(v4 ? k_dn_chunk_out<true> : k_dn_chunk_out<false>, dim3(nch, H), dim3(256), 0,
-                       st, w.qn, w.vv, w.Mq, w.U, w.Gc, proj, ldp, T, norm_w, out, ldo, H,
-                       conv_state, p0);
+    // up to two workgroups a CU a chunk's row blocks go to four workgroups, which
+    // read its state four times (16 heads: 300 rows 12.5 us split; 600 rows, 640
+    // workgroups split, 16.2 us whole and 16.6 split)
+    const bool split = nch * H * 4 <= 512;
+    const auto kern = split ? (v4 ? k_dn_chunk_out<1, true> : k_dn_chunk_out<1, false>)
+                            : (v4 ? k_dn_chunk_out<4, true> : k_dn_chunk_out<4, false>);
+    hipLaunchKernelGGL(kern, dim3(nch * (split ? 4 : 1), H), dim3(256), 0, st, w.qn, w.vv, w.Mq, w.U,
+                       w.Gc, proj, ldp, T, norm_w, out, ldo, H, conv_state, p0);
     return qlm_launch_status();
 }
 
