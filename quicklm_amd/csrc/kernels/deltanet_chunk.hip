@@ -16,7 +16,7 @@
 // Every decay factor is exp of a non-positive number (ratios, never 1/gamma).
 //
 // Kernels (one stream, in order):
-//   k_dn_chunk_prep   per (16 rows, head): conv taps from the prompt rows or
+//   k_dn_chunk_prep   per (8 or 16 rows, head): conv taps from the prompt rows or
 //                     the ring (positions before p0), SiLU, L2 norms, gates --
 //                     the decode step's arithmetic;
 //   k_dn_chunk_intra  per (chunk, head): everything that does not depend on
@@ -74,21 +74,23 @@ __device__ __forceinline__ size_t gix(int t, int h, int H) {
 }
 __device__ __forceinline__ size_t rix(int t, int h, int H) { return gix(t, h, H) * kD; }
 
-// Rows a prep or post workgroup handles (a conv window slides down them).
-constexpr int kPR = 16;
-
-// Per (16 rows, head): thread (section, column) slides the conv window down
+// Per (PR rows, head): thread (section, column) slides the conv window down
 // the rows, the q and k outputs wait in LDS for their row norms (6 waves, a
-// norm each at a time), v goes straight out.
+// norm each at a time), v goes straight out. 16 heads, us at 4 / 8 / 16 / 32
+// rows a workgroup: 66 rows 5.0 / 5.0 / 7.7 / 12.4, 300 rows 9.2 / 8.9 / 10.9 /
+// 12.9, 700 rows 16.6 / 14.6 / 14.7 / 19.9, 2047 rows 38.6 / 32.2 / 32.0 / 33.2
+// (there bound by the vector work of the SiLUs and divisions as much as by its
+// 100 MB): 8 rows while the workgroups are few, 16 above.
+template <int PR>
 __global__ __launch_bounds__(3 * kD) void k_dn_chunk_prep(
     const float* __restrict__ proj, int ldp, int T, const float* __restrict__ conv_state,
     const float* __restrict__ wt, const float* __restrict__ A_log,
     const float* __restrict__ dt_bias, int p0, int H, float* __restrict__ qn,
     float* __restrict__ kn, float* __restrict__ vv, float* __restrict__ alpha,
     float* __restrict__ beta) {
-    __shared__ float ys[2][kPR][kD];
-    const int t0 = blockIdx.x * kPR, h = blockIdx.y, tid = threadIdx.x;
-    const int nt = min(kPR, T - t0);
+    __shared__ float ys[2][PR][kD];
+    const int t0 = blockIdx.x * PR, h = blockIdx.y, tid = threadIdx.x;
+    const int nt = min(PR, T - t0);
     const int lane = tid & 63, wave = tid >> 6;
     const int HD = H * kD, C = 3 * HD;
     const int sec = tid / kD, tt = tid % kD, ch = sec * HD + h * kD + tt;
@@ -108,11 +110,11 @@ __global__ __launch_bounds__(3 * kD) void k_dn_chunk_prep(
             xw[j] = conv_state[(size_t)row * C + ch];
         }
     }
-    float xr[kPR];  // rows past T read row T-1 and are never stored
+    float xr[PR];  // rows past T read row T-1 and are never stored
 #pragma unroll
-    for (int r = 0; r < kPR; ++r) xr[r] = proj[(size_t)min(t0 + r, T - 1) * ldp + ch];
+    for (int r = 0; r < PR; ++r) xr[r] = proj[(size_t)min(t0 + r, T - 1) * ldp + ch];
 #pragma unroll
-    for (int r = 0; r < kPR; ++r) {
+    for (int r = 0; r < PR; ++r) {
         float acc = 0.0f;
         acc = nc_add_mul(acc, xw[0], w0);
         acc = nc_add_mul(acc, xw[1], w1);
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(3 * kD) void k_dn_chunk_prep(
         beta[gix(t, h, H)] = 1.0f / (1.0f + expf(-pr[4 * HD + h]));
     }
     __syncthreads();
-    for (int i = wave; i < 2 * kPR; i += 3 * kD / 64) {
+    for (int i = wave; i < 2 * PR; i += 3 * kD / 64) {
         const int which = i & 1, r = i >> 1;
         if (r >= nt) break;
         const float a0 = ys[which][r][lane], a1 = ys[which][r][lane + 64];
@@ -663,8 +665,9 @@ extern "C" int qlm_deltanet_prefill_chunked(const float* proj, int ldp, int T, f
     if (work_bytes < w.bytes || ((uintptr_t)work & 255u)) return QLM_ERR_ARG;
     hipStream_t st = as_stream(stream);
     const int nch = (T + kC - 1) / kC;
-    const int nrb = (T + kPR - 1) / kPR;
-    hipLaunchKernelGGL(k_dn_chunk_prep, dim3(nrb, H), dim3(3 * kD), 0, st, proj, ldp, T, conv_state,
+    const bool few = (long long)T * H < 8192;
+    hipLaunchKernelGGL(few ? k_dn_chunk_prep<8> : k_dn_chunk_prep<16>,
+                       dim3(few ? (T + 7) / 8 : (T + 15) / 16, H), dim3(3 * kD), 0, st, proj, ldp, T, conv_state,
                        conv_w_t, A_log, dt_bias, p0, H, w.qn, w.kn, w.vv, w.alpha, w.beta);
     int rc = qlm_launch_status();
     if (rc != QLM_OK) return rc;
@@ -694,5 +697,5 @@ extern "C" int qlm_deltanet_prefill_chunked(const float* proj, int ldp, int T, f
 // measured inside a first prefill or decode step).
 hipError_t qlm_load_deltanet_chunk() {
     hipFuncAttributes a;
-    return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(k_dn_chunk_prep));
+    return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(k_dn_chunk_chain));
 }
