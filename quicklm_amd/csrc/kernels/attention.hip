@@ -624,8 +624,11 @@ __global__ __launch_bounds__(kThreads) void k_gqa_prep_rows(
 // Lane (qd, n) ends with row n's outputs 16 c + 4 qd .. + 3 for c = 0..7.
 // Keys past the workgroup's last position are clamped to it (probability 0;
 // the cache beyond is not written yet). A value that is not finite goes whole
-// into the l term, which only meets the other side's h, so it acts as it
-// would in an fp32 product.
+// into the l term, which only meets the other side's h: what it makes is not
+// finite either, but can be NaN where an fp32 product is infinite (two such
+// values) and reaches rows that do not see the key (probability 0, in a block
+// of 32 keys they share). So an output that comes out not finite is computed
+// again in the fp32 form (f32_tile) and replaced; the others stay.
 // gridDim.z > 1 splits the keys in ranges of `ch` and leaves k_attn's record
 // [m, l, -, -, o] per (row, head, range) for k_attn_combine: a few rows over
 // a long context would otherwise walk it on a handful of workgroups.
@@ -662,8 +665,9 @@ __device__ __forceinline__ Split8 split8_finite(const float (&x)[8]) {
     return s;
 }
 
-// the same for any floats: one that is not finite, or would round to
-// infinity, is left whole (truncated to bf16) in the l term
+// the same for any floats: a finite one that would round to infinity has its h
+// truncated (the rest then takes 16 bits: still exact); one that is not finite
+// is left whole (truncated to bf16) in the l term
 __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
     Split8 s = split8_finite(x);
     unsigned top = 0;
@@ -673,13 +677,19 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const unsigned u = __float_as_uint(x[i]), a = u & 0x7fffffffu;
-            const unsigned half = 0xffffu << (16 * (i & 1));
-            const unsigned whole = (u >> 16) | (a > 0x7f800000u ? 0x40u : 0u);
-            if (a >= 0x7f7f8000u) {
-                s.t[0][i / 2] &= ~half;
-                s.t[1][i / 2] &= ~half;
-                s.t[2][i / 2] = (s.t[2][i / 2] & ~half) | (whole << (16 * (i & 1)));
+            if (a < 0x7f7f8000u) continue;
+            unsigned t[3] = {0u, 0u, (u >> 16) | (a > 0x7f800000u ? 0x40u : 0u)};
+            if (a < 0x7f800000u) {
+                const float r = x[i] - __uint_as_float(u & 0xffff0000u);
+                t[0] = u >> 16;
+                t[1] = __builtin_bit_cast(unsigned short, (__bf16)r);
+                t[2] = __builtin_bit_cast(unsigned short,
+                                          (__bf16)(r - __uint_as_float(t[1] << 16)));
             }
+            const int sh = 16 * (i & 1);
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                s.t[k][i / 2] = (s.t[k][i / 2] & ~(0xffffu << sh)) | (t[k] << sh);
         }
     }
     return s;
@@ -695,6 +705,102 @@ __device__ __forceinline__ f32x4 mfma_bf16(pf_u32x4 a, pf_u32x4 b, f32x4 c) {
 
 // 2^x for x <= 0 by v_exp_f32 (1 ulp)
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
+
+__device__ __forceinline__ bool finite4(f32x4 v) {
+    const f32x4 z = v * 0.0f;  // NaN for one that is not
+    return (z[0] + z[1]) + (z[2] + z[3]) == 0.0f;
+}
+
+// ---- the fp32 form: 16 query rows x 16 keys on v_mfma_f32_16x16x4f32 ----
+//
+// A lane l: row l % 16, k l / 16; B lane l: k l / 16, column l % 16; D lane l:
+// rows 4 (l / 16) .. +3, column l % 16:
+//   S^T = K Q^T: A = 16 keys, B = Q^T of the wave's 16 rows, the head's 128
+//     elements split as 32 k-steps of element 32 (l / 16) + s, so a lane
+//     loads 32 contiguous floats of its key (kd) and of its query row (qv);
+//     lane (qd, n) then holds the scores of row n for keys 4 qd .. 4 qd + 3;
+//   O^T += V^T P^T: k-step j takes keys 4 qd + j, which is where those
+//     scores already are, so the probabilities feed the B operand from the
+//     registers that computed them; A lane (qd, n) reads V[key][16 c + n] (vd).
+// Lane (qd, n) ends with row n's outputs 16 c + 4 qd .. + 3 for c = 0..7.
+// RANGE: the keys may begin past a row's own position.
+struct F32Rows {
+    f32x4 o[8];
+    float m, l;
+};
+
+__device__ __forceinline__ void f32_load32(float (&d)[32], const float* p) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(p + 4 * j);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[4 * j + i] = x[i];
+    }
+}
+
+template <bool RANGE>
+__device__ __forceinline__ void f32_keys(F32Rows& a, const float (&kd)[32],
+                                         const float (&vd)[4][8], const float (&qv)[32], int key0,
+                                         int qpos, float scale) {
+    // S^T: two independent chains over the 32 k-steps
+    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 32; s += 2) {
+        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kd[s], qv[s], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kd[s + 1], qv[s + 1], s1, 0, 0, 0);
+    }
+    float sc[4], tm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        sc[i] = key0 + i <= qpos ? (s0[i] + s1[i]) * scale : -INFINITY;
+        tm = fmaxf(tm, sc[i]);
+    }
+    // the row's maximum over the 16 keys (lanes n, n+16, n+32, n+48)
+    const float mn = fmaxf(a.m, cols_max(tm));
+    const float mref = RANGE && mn == -INFINITY ? 0.0f : mn;
+    const float alpha = expf(a.m - mref);  // 0 on the first tile
+    float p[4], ps = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        p[i] = expf(sc[i] - mref);
+        ps += p[i];
+    }
+    a.l = fmaf(a.l, alpha, cols_sum(ps));
+    a.m = mn;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) a.o[c] *= alpha;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            a.o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vd[j][c], p[j], a.o[c], 0, 0, 0);
+}
+
+// One wave: the 16 rows of query row pointer qr (this lane's) over keys
+// kbeg .. last of a kv head whose K and V begin at kp and vp.
+__device__ __forceinline__ F32Rows f32_tile(const float* qr, const float* kp, const float* vp,
+                                            size_t kstride, int kbeg, int last, int qpos,
+                                            float scale) {
+    const int lane = threadIdx.x & (QLM_WAVE - 1), qd = lane >> 4, n = lane & 15;
+    F32Rows a;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) a.o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    a.m = -INFINITY, a.l = 0.0f;
+    float qv[32];
+    f32_load32(qv, qr + 32 * qd);
+#pragma unroll 1
+    for (int k0 = kbeg; k0 <= last; k0 += 16) {
+        float kd[32], vd[4][8];
+        f32_load32(kd, kp + min(k0 + n, last) * kstride + 32 * qd);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                vd[j][c] = vp[min(k0 + 4 * qd + j, last) * kstride + 16 * c + n];
+        f32_keys<true>(a, kd, vd, qv, k0 + 4 * qd, qpos, scale);
+    }
+    return a;
+}
 
 template <int G>
 struct PfShape {
@@ -1012,41 +1118,71 @@ __global__ __launch_bounds__(PfShape<G>::NTH, 2) void k_attn_pf(
                 o[r][c >> 2][c & 3] = o[r][c >> 2][c & 3] * f0 + mg[r][at * RS + c] * f1;
         }
     }
+    // where elements 16 c + 4 qd .. + 3 of row t go (record or output), and what
+    // becomes of them on the way
+    auto record = [&](int t) {
+        return work +
+               (((size_t)t * (gridDim.y * G) + h) * gridDim.z + blockIdx.z) * (HD + 4);
+    };
+    auto place = [&](int t, int c) {
+        return reinterpret_cast<f32x4*>(work ? record(t) + 4 + 16 * c + 4 * qd
+                                             : out + (size_t)t * ldo + (size_t)h * HD + 16 * c +
+                                                   4 * qd);
+    };
+    auto gate = [&](int t, int c, f32x4 y) {
+        if (gated && !work) {
+            const f32x4 gg = *reinterpret_cast<const f32x4*>(
+                qkv + (size_t)t * ldq + (size_t)h * qhs + HD + 16 * c + 4 * qd);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] /= 1.0f + expf(-gg[i]);
+        }
+        return y;
+    };
+    bool odd[2] = {false, false};
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
         const int tq = t0[r] + n;
         if (last[r] < kbeg || tq >= T) continue;
+        float f;
         if (work) {
             // the record's maximum is in natural units; what its rounding
             // changes goes into l and o
             const float mr = m[r] * 0.69314718f;
             float e = fmaf(-mr, 1.44269502f, m[r]);
             e = m[r] == -INFINITY ? 0.0f : fmaf(-mr, 1.92596303e-8f, e);
-            const float f = exp2_fast(e);
-            float* rec = work + (((size_t)tq * (gridDim.y * G) + h) * gridDim.z + blockIdx.z) *
-                                    (HD + 4);
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-                *reinterpret_cast<f32x4*>(rec + 4 + 16 * c + 4 * qd) = o[r][c] * f;
+            f = exp2_fast(e);
             if (qd == 0) {
-                rec[0] = mr;
-                rec[1] = l[r] * f;
+                record(tq)[0] = mr;
+                record(tq)[1] = l[r] * f;
             }
-            continue;
+        } else {
+            f = 1.0f / l[r];
         }
-        const float* grow = qkv + (size_t)tq * ldq + (size_t)h * qhs + HD;
-        float* dst = out + (size_t)tq * ldo + (size_t)h * HD;
-        const float inv = 1.0f / l[r];
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            const int e = 16 * c + 4 * qd;
-            f32x4 y = o[r][c] * inv;
-            if (gated) {
-                const f32x4 gg = *reinterpret_cast<const f32x4*>(grow + e);
+            const f32x4 y = gate(tq, c, o[r][c] * f);
+            *place(tq, c) = y;
+            odd[r] |= !finite4(y);
+        }
+    }
+#pragma unroll 1
+    for (int r = 0; r < 2; ++r) {
+        const bool mine = r ? odd[1] : odd[0];
+        if (!__any(mine)) continue;
+        const int tq = max(0, min((r ? t0[1] : t0[0]) + n, T - 1));
+        const F32Rows a = f32_tile(qkv + (size_t)tq * ldq + (size_t)h * qhs,
+                                   kc + (size_t)g * HD, vc + (size_t)g * HD, kstride, kbeg,
+                                   min(r ? last[1] : last[0], kend - 1), p0 + tq,
+                                   qscale * 0.69314718f);
+        if (!mine) continue;
+        const float f = work ? expf(a.m - (r ? m[1] : m[0]) * 0.69314718f) : 1.0f / a.l;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) y[i] /= 1.0f + expf(-gg[i]);
-            }
-            *reinterpret_cast<f32x4*>(dst + e) = y;
+        for (int c = 0; c < 8; ++c) {
+            f32x4 y = *place(tq, c);
+            const f32x4 z = gate(tq, c, a.o[c] * f);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = y[i] * 0.0f == 0.0f ? y[i] : z[i];
+            *place(tq, c) = y;
         }
     }
 }
@@ -1060,17 +1196,7 @@ __global__ __launch_bounds__(PfShape<G>::NTH, 2) void k_attn_pf(
 // 41 against 38): a workgroup owns 16 consecutive prompt rows and one kv head, wave w the query
 // head g G + w, and walks the keys 0 .. (its last row's position) in tiles of
 // 16 with an online softmax per row (attention.cpp:54-82 per row: the scores
-// q . k / sqrt(hd), softmax, the weighted sum of V). Both products run on
-// v_mfma_f32_16x16x4f32 (A lane l: row l % 16, k l / 16; B lane l: k l / 16,
-// column l % 16; D lane l: rows 4 (l / 16) .. +3, column l % 16):
-//   S^T = K Q^T: A = 16 keys, B = Q^T of the wave's 16 rows, the head's 128
-//     elements split as 32 k-steps of element 32 (l / 16) + s, so a lane
-//     loads 32 contiguous floats of its key (and of its query row, once);
-//     lane (qd, n) then holds the scores of row n for keys 4 qd .. 4 qd + 3;
-//   O^T += V^T P^T: k-step j takes keys 4 qd + j, which is where those
-//     scores already are, so the probabilities feed the B operand from the
-//     registers that computed them; A lane (qd, n) reads V[key][16 c + n].
-// Lane (qd, n) ends with row n's outputs 16 c + 4 qd .. + 3 for c = 0..7.
+// q . k / sqrt(hd), softmax, the weighted sum of V), f32_keys a tile.
 // Key rows past the tile's last position are clamped to it (their
 // probabilities are 0 and the cache beyond is not written yet).
 template <int G>
@@ -1092,22 +1218,11 @@ __global__ __launch_bounds__(G * QLM_WAVE) void k_attn_pf_few(const float* __res
     const int ntiles = last / 16 + 1;
 
     float qv[32];
-    {
-        const float4* qr =
-            reinterpret_cast<const float4*>(qkv + (size_t)tq * ldq + (size_t)h * qhs + 32 * qd);
+    f32_load32(qv, qkv + (size_t)tq * ldq + (size_t)h * qhs + 32 * qd);
+    F32Rows a;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float4 x = qr[j];
-            qv[4 * j] = x.x;
-            qv[4 * j + 1] = x.y;
-            qv[4 * j + 2] = x.z;
-            qv[4 * j + 3] = x.w;
-        }
-    }
-    f32x4 o[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.0f;
+    for (int c = 0; c < 8; ++c) a.o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    a.m = -INFINITY, a.l = 0.0f;
     const size_t kstride = (size_t)n_kv * HD;
 
     // The workgroup stages each 16-key tile of K and V once in LDS (rows
@@ -1143,54 +1258,12 @@ __global__ __launch_bounds__(G * QLM_WAVE) void k_attn_pf_few(const float* __res
         const int k0 = kt * 16, buf = kt & 1;
         // K row n of the tile, elements 32 qd .. + 31; V[key 4 qd + j][16 c + n]
         float kd[32], vd[4][8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float4 x = *reinterpret_cast<const float4*>(&kvs[buf][0][n * RS + 32 * qd + 4 * j]);
-            kd[4 * j] = x.x;
-            kd[4 * j + 1] = x.y;
-            kd[4 * j + 2] = x.z;
-            kd[4 * j + 3] = x.w;
-        }
+        f32_load32(kd, &kvs[buf][0][n * RS + 32 * qd]);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int c = 0; c < 8; ++c) vd[j][c] = kvs[buf][1][(4 * qd + j) * RS + 16 * c + n];
-        // S^T: two independent chains over the 32 k-steps
-        f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < 32; s += 2) {
-            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kd[s], qv[s], s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kd[s + 1], qv[s + 1], s1, 0, 0, 0);
-        }
-        float sc[4], tm = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int key = k0 + 4 * qd + i;
-            sc[i] = key <= qpos ? (s0[i] + s1[i]) * scale : -INFINITY;
-            tm = fmaxf(tm, sc[i]);
-        }
-        // the row's maximum over the 16 keys (lanes n, n+16, n+32, n+48)
-        tm = cols_max(tm);
-        const float mn = fmaxf(m, tm);
-        const float alpha = expf(m - mn);  // 0 on the first tile
-        float p[4], ps = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            p[i] = expf(sc[i] - mn);
-            ps += p[i];
-        }
-        ps = cols_sum(ps);
-        l = fmaf(l, alpha, ps);
-        m = mn;
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o[c][i] *= alpha;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-                o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vd[j][c], p[j], o[c], 0, 0, 0);
+        f32_keys<false>(a, kd, vd, qv, k0 + 4 * qd, qpos, scale);
         stage(buf ^ 1);  // past the end: a copy of the last tile nobody reads
         fetch(min(k0 + 32, 16 * (ntiles - 1)));
         __syncthreads();
@@ -1202,7 +1275,7 @@ __global__ __launch_bounds__(G * QLM_WAVE) void k_attn_pf_few(const float* __res
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
         const int e = 16 * c + 4 * qd;
-        float r[4] = {o[c][0] / l, o[c][1] / l, o[c][2] / l, o[c][3] / l};
+        float r[4] = {a.o[c][0] / a.l, a.o[c][1] / a.l, a.o[c][2] / a.l, a.o[c][3] / a.l};
         if (gated) {
             const float4 gg = *reinterpret_cast<const float4*>(grow + e);
             r[0] *= 1.0f / (1.0f + expf(-gg.x));

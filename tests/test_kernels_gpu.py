@@ -880,6 +880,64 @@ def test_gqa_prefill_split_terms(hip, orc, rng, n_q, n_kv, p0, T):
         assert np.array_equal(again, got)
 
 
+@pytest.mark.parametrize("n_q,n_kv,p0,T,max_seq", [
+    (16, 4, 3, 100, 700),                         # the few-key form
+    (8, 8, 150, 60, 700), (8, 4, 200, 45, 700),   # key ranges merged
+    (16, 4, 70, 290, 700), (16, 2, 37, 250, 700),  # keys split by each workgroup
+    (16, 4, 0, 304, 2048), (16, 4, 37, 600, 2048), (16, 2, 0, 272, 700)])  # split planes
+def test_gqa_prefill_values_not_finite(hip, orc, rng, n_q, n_kv, p0, T, max_seq):
+    """An infinite or NaN V element of a prompt row reaches the rows of its
+    16-row tile and later ones (a masked key of the tile is multiplied by
+    probability 0), never a tile before it: those rows stay within the fp32
+    attention's bar (1e-5), every other column keeps its bits. V elements at
+    the top of the fp32 range keep all their bits (same bar)."""
+    hd, rot, theta, gated = 128, 32, 1e6, 1
+    ld, kv = n_q * 2 * hd + 2 * n_kv * hd, n_kv - 1
+    qn = (rng.standard_normal(hd) * 0.02).astype(np.float32)
+    kn = (rng.standard_normal(hd) * 0.02).astype(np.float32)
+    cos_t, sin_t = orc.rope_table(theta, rot, max_seq)
+    kc = np.zeros((max_seq, n_kv, hd), np.float32)
+    vc = np.zeros_like(kc)
+    kc[:p0] = rng.standard_normal((p0, n_kv, hd))
+    vc[:p0] = rng.standard_normal((p0, n_kv, hd))
+    qkv = rng.standard_normal((T, ld)).astype(np.float32)
+    nwork = hip.lib().qlm_gqa_prefill_workspace_bytes(n_q, hd, max_seq)
+
+    def run(rows):
+        work = hip.DeviceBuffer(nwork)
+        do = hip.DeviceBuffer(T * n_q * hd * 4)
+        say("gqa_prefill values not finite", n_q, n_kv, p0, T, max_seq)
+        hip.call("qlm_gqa_prefill", dev(hip, rows), ld, dev(hip, qn), dev(hip, kn),
+                 dev(hip, cos_t), dev(hip, sin_t), rot, dev(hip, kc), dev(hip, vc), max_seq,
+                 p0, T, do, n_q * hd, n_q, n_kv, hd, gated, work, None)
+        return do.to_numpy((T, n_q, hd), np.float32)
+
+    v0 = ld - (n_kv - kv) * hd  # first V column of that kv head
+    G = n_q // n_kv
+    heads = slice(kv * G, (kv + 1) * G)
+    clean = run(qkv)
+    bad = qkv.copy()
+    tiles = range(1, (T + 15) // 16)
+    for j in tiles:  # column j: the first row of tile j
+        bad[16 * j, v0 + j] = (np.inf, -np.inf, np.nan)[j % 3]
+    got = run(bad)
+    for j in tiles:
+        assert rel_err(got[:16 * j, heads, j], clean[:16 * j, heads, j]) < 1e-5, j
+        assert not np.isfinite(got[16 * j:, heads, j]).any()
+        got[:, heads, j] = clean[:, heads, j]
+    assert np.array_equal(got, clean)
+
+    top = qkv.copy()  # above the largest bf16, not exact in 8 bits
+    top[0, v0 + 5], top[T // 2, v0 + 9] = 3.4e38, -3.3977e38
+    kref, vref = kc.copy(), vc.copy()
+    ref = np.stack([orc.gqa_core(top[t].copy(), qn, kn, theta, rot, kref, vref, p0 + t, n_q, n_kv,
+                                 hd, gated).reshape(n_q, hd) for t in range(T)])
+    got = run(top)
+    for c, t in ((5, 0), (9, T // 2)):
+        scale = np.float32(2.0 ** -100)  # the norms' squares stay in range
+        assert rel_err(got[t:, heads, c] * scale, ref[t:, heads, c] * scale) < 1e-5
+
+
 # ---------------------------------------------------------------- A8/A9 GQA
 @pytest.mark.parametrize("n_q,n_kv,hd,rot,gated,max_seq,start",
                          [(16, 4, 128, 32, 1, 600, (300, 511)),
