@@ -190,7 +190,8 @@ int qlm_gemv_mx_l2_plan(const void* q_tiles, const float* s_tiles, int group, in
  * contents needed; calls that share it must be ordered on one stream). More
  * than 64 rows split K over workgroups where that fills the GPU; with less
  * workspace, down to 4 M + 4 M K bytes (each term rounded up to 256), they
- * take the slices whose sums fit. The size never falls with M. */
+ * take the slices whose sums fit. The size never falls with M: a workspace
+ * for the most rows serves every call of fewer. */
 size_t qlm_matmul_i8_workspace_bytes(int M, int N, int K, int epilogue);
 
 int qlm_matmul_i8(const float* x, int ldx, const float* norm_w, float eps, const int8_t* q,

@@ -18,6 +18,8 @@
 // an activation split once per call. Epilogues: store, residual add, SwiGLU
 // (weights [2F, K]: silu(gate) * up formed in registers).
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "mm_reduce.hpp"
 
@@ -1219,7 +1221,12 @@ int mm_run(const float* x, int ldx, float* rs, const float* nw, float eps, const
 
 extern "C" size_t qlm_matmul_i8_workspace_bytes(int M, int N, int K, int epilogue) {
     if (M <= 0 || N <= 0 || K <= 0 || epilogue < EPI_STORE || epilogue > EPI_SWIGLU) return 0;
-    return mm_workspace(M, N, K, epilogue, true);
+    // 16 and 64 rows are the last of a K-slice rule and can need more than the
+    // rows after them (64: 50 MB, 65: 35 MB for a gate/up of 2 x 9728 x 2560)
+    size_t b = mm_workspace(M, N, K, epilogue, true);
+    for (const int m : {16, 64})
+        if (m < M) b = std::max(b, mm_workspace(m, N, K, epilogue, true));
+    return b;
 }
 
 extern "C" size_t qlm_matmul_bf16_workspace_bytes(int M, int K) {

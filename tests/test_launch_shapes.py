@@ -79,3 +79,16 @@ def test_matmul_mx_shapes(M):
     assert served > 50
     assert lib.qlm_matmul_i8_mx_shape(17, 2560, 2560, 0, C.byref(w), C.byref(u), C.byref(r),
                                       C.byref(g)) == -2
+
+
+@pytest.mark.parametrize("N,K", [(9728, 2560), (2560, 9728), (8224, 2560), (2560, 2048),
+                                 (3584, 1024), (32768, 1024), (151936, 2560), (255, 64),
+                                 (300, 96), (256, 1088), (4096, 4096), (1000, 12288)])
+def test_matmul_i8_workspace_grows_with_rows(N, K):
+    """A workspace sized for the most rows serves fewer: the query never falls
+    from M to M + 1 (K on and off the multiples of 128, every epilogue)."""
+    lib = hip.lib()
+    for epi in (0, 1, 2):
+        sizes = [lib.qlm_matmul_i8_workspace_bytes(M, N, K, epi) for M in range(1, 301)]
+        falls = [M for M in range(1, 300) if sizes[M] < sizes[M - 1]]
+        assert not falls, (epi, falls)
