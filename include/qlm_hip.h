@@ -445,9 +445,22 @@ int qlm_gqa_decode(float* qkv, int ldqkv, const float* q_norm, const float* k_no
  * reference's batched forward (attention.cpp:138-232 per row). q rows are
  * normalised and rotated in place; k/v rows go to the cache of that sequence
  * (k_cache, v_cache point at its [max_seq, n_kv, hd] block) before any row
- * attends. out[t] is [n_q*hd] (row stride ldo). work is
- * qlm_gqa_prefill_workspace_bytes(n_q, hd, max_seq) bytes. */
+ * attends. out[t] is [n_q*hd] (row stride ldo). work is device scratch of
+ * qlm_gqa_prefill_workspace_bytes(n_q, hd, max_seq) bytes (of the call's own
+ * max_seq; no initial contents needed): every form but the few-key one may
+ * write all of it (the rows' partial results, and the keys split for the
+ * matrix cores), so calls that share it must be ordered on one stream. 16-byte
+ * aligned; with hd 128 and row strides that are multiples of 4 a buffer of
+ * less alignment is accepted and left unused (slower). */
 size_t qlm_gqa_prefill_workspace_bytes(int n_q, int hd, int max_seq);
+
+/* What such a call runs (work aligned, row strides multiples of 4; host only,
+ * no counterpart in the reference): form 0: records a chunk of keys, merged
+ * (hd 256); 1: the few-key form; 2: keys split by each workgroup; 3: keys
+ * split once beforehand. ranges: key ranges merged afterwards (1: none);
+ * bytes: of `work` that are written. */
+int qlm_gqa_prefill_plan(int n_q, int n_kv, int hd, int max_seq, int p0, int T, int* form,
+                         int* ranges, size_t* bytes);
 int qlm_gqa_prefill(float* qkv, int ldqkv, const float* q_norm, const float* k_norm,
                     const float* cos_tab, const float* sin_tab, int rot_dim, float* k_cache,
                     float* v_cache, int max_seq, int p0, int T, float* out, int ldo, int n_q,

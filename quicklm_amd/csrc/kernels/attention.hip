@@ -1850,19 +1850,22 @@ namespace {
 // launch would leave most of the chip idle; then as many as bring it to ~256
 // workgroups, at least 64 keys each, and no more records than the workspace
 // holds. Split planes (k_pf_split): for G >= 4 and enough rows, where the
-// workspace has room for them before the records.
+// workspace has room for them before the records. Without the workspace
+// (use_work false: not 16-byte aligned, as planes and records are written)
+// one range and no planes, which need none.
 struct PfPlan {
     int groups, ranges, ch;
     bool planes;
     size_t rec_at;  // floats from the workspace's start to the records
+    size_t bytes;   // of the workspace that are written
 };
-PfPlan prefill_plan(int G, int n_q, int n_kv, int p0, int T, int max_seq) {
+PfPlan prefill_plan(int G, int n_q, int n_kv, int p0, int T, int max_seq, bool use_work) {
     const int rg = G >= 4 ? 1 : 4 / G;
     const int slots = ((T + 15) / 16 + 1) / 2;
     PfPlan p;
     p.groups = (slots + rg - 1) / rg;
     const int keys = p0 + T;
-    const size_t bytes = records_bytes(kPrefillSlice, n_q, 128, max_seq, kNtLong);
+    const size_t bytes = use_work ? records_bytes(kPrefillSlice, n_q, 128, max_seq, kNtLong) : 0;
     const size_t row = (size_t)n_q * (128 + 4) * sizeof(float);  // a row's records, one range
     const size_t pl = (size_t)n_kv * ((keys + 31) / 32) * 2 * kPfUnits * 16;
     int z = 256 / (p.groups * n_kv);
@@ -1874,6 +1877,7 @@ PfPlan prefill_plan(int G, int n_q, int n_kv, int p0, int T, int max_seq) {
     p.ranges = (keys + p.ch - 1) / p.ch;
     p.planes = G >= 4 && T >= kPfPlaneRows && pl + (p.ranges > 1 ? row * T * p.ranges : 0) <= bytes;
     p.rec_at = p.planes ? pl / sizeof(float) : 0;
+    p.bytes = (p.planes ? pl : 0) + (p.ranges > 1 ? row * T * p.ranges : 0);
     return p;
 }
 
@@ -1882,6 +1886,30 @@ PfPlan prefill_plan(int G, int n_q, int n_kv, int p0, int T, int max_seq) {
 extern "C" size_t qlm_gqa_prefill_workspace_bytes(int n_q, int hd, int max_seq) {
     if (n_q <= 0 || hd <= 0 || max_seq <= 0) return 0;
     return records_bytes(kPrefillSlice, n_q, hd, max_seq, kNtLong);
+}
+
+extern "C" int qlm_gqa_prefill_plan(int n_q, int n_kv, int hd, int max_seq, int p0, int T,
+                                    int* form, int* ranges, size_t* bytes) {
+    if (!form || !ranges || !bytes) return QLM_ERR_ARG;
+    if (T <= 0 || p0 < 0 || n_q <= 0 || n_kv <= 0 || max_seq <= 0) return QLM_ERR_ARG;
+    if (p0 + T > max_seq || n_q % n_kv != 0 || (hd != 128 && hd != 256)) return QLM_ERR_SHAPE;
+    const int G = n_q / n_kv;
+    if (G != 1 && G != 2 && G != 4 && G != 8) return QLM_ERR_SHAPE;
+    *ranges = 1;
+    *bytes = 0;
+    if (hd != 128) {
+        *form = 0;
+        *ranges = nchunks_for(max_seq, chunk_len(hd, kNtLong));
+        *bytes = qlm_gqa_prefill_workspace_bytes(n_q, hd, max_seq);
+    } else if (p0 + T <= kPfFewKeys) {
+        *form = 1;
+    } else {
+        const PfPlan p = prefill_plan(G, n_q, n_kv, p0, T, max_seq, true);
+        *form = p.planes ? 3 : 2;
+        *ranges = p.ranges;
+        *bytes = p.bytes;
+    }
+    return QLM_OK;
 }
 
 extern "C" int qlm_gqa_prefill(float* qkv, int ldqkv, const float* q_norm, const float* k_norm,
@@ -1931,7 +1959,7 @@ extern "C" int qlm_gqa_prefill(float* qkv, int ldqkv, const float* q_norm, const
             QLM_ATTN_FEW(8)
 #undef QLM_ATTN_FEW
         }
-        const PfPlan pl = prefill_plan(G, n_q, n_kv, p0, T, max_seq);
+        const PfPlan pl = prefill_plan(G, n_q, n_kv, p0, T, max_seq, ((uintptr_t)work & 15u) == 0);
         float* rec = pl.ranges > 1 ? w + pl.rec_at : nullptr;
         pf_u32x4* planes = reinterpret_cast<pf_u32x4*>(work);
         if (pl.planes) {

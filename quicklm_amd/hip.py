@@ -63,6 +63,8 @@ _SIGS = {
     "qlm_deltanet_prefill_chunked": (_i, [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i,
                                           _i, _i, _vp, _sz, _vp]),
     "qlm_gqa_prefill_workspace_bytes": (_sz, [_i, _i, _i]),
+    "qlm_gqa_prefill_plan": (_i, [_i, _i, _i, _i, _i, _i, C.POINTER(_i), C.POINTER(_i),
+                                  C.POINTER(_sz)]),
     "qlm_gqa_prefill": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _vp, _i, _i,
                              _i, _i, _i, _vp, _vp]),
     "qlm_matmul_i8_workspace_bytes": (_sz, [_i, _i, _i, _i]),

@@ -938,6 +938,39 @@ def test_gqa_prefill_values_not_finite(hip, orc, rng, n_q, n_kv, p0, T, max_seq)
         assert rel_err(got[t:, heads, c] * scale, ref[t:, heads, c] * scale) < 1e-5
 
 
+@pytest.mark.parametrize("n_q,n_kv,p0,T", [(16, 4, 600, 5), (16, 4, 20, 320), (8, 8, 150, 60)])
+@pytest.mark.parametrize("shift", [4, 8])
+def test_gqa_prefill_workspace_alignment(hip, orc, rng, n_q, n_kv, p0, T, shift):
+    """A workspace that is not 16-byte aligned is accepted and left unused:
+    one key range, keys split by each workgroup. Within the fp32 attention's
+    bar (1e-5) of the same call with an aligned one."""
+    hd, rot, max_seq, theta, gated = 128, 32, 2048, 1e6, 1
+    ld = n_q * 2 * hd + 2 * n_kv * hd
+    gain = (rng.standard_normal(hd) * 0.02).astype(np.float32)
+    cos_t, sin_t = orc.rope_table(theta, rot, max_seq)
+    kc = rng.standard_normal((max_seq, n_kv, hd)).astype(np.float32)
+    vc = rng.standard_normal((max_seq, n_kv, hd)).astype(np.float32)
+    qkv = rng.standard_normal((T, ld)).astype(np.float32)
+    nwork = hip.lib().qlm_gqa_prefill_workspace_bytes(n_q, hd, max_seq)
+    fill = np.full(nwork + 16, 0x5A, np.uint8)
+
+    def run(by):
+        work = hip.DeviceBuffer(nwork + 16)
+        work.upload(fill)
+        do = hip.DeviceBuffer(T * n_q * hd * 4)
+        say("gqa_prefill workspace alignment", n_q, n_kv, p0, T, by)
+        hip.call("qlm_gqa_prefill", dev(hip, qkv), ld, dev(hip, gain), dev(hip, gain),
+                 dev(hip, cos_t), dev(hip, sin_t), rot, dev(hip, kc), dev(hip, vc), max_seq,
+                 p0, T, do, n_q * hd, n_q, n_kv, hd, gated, work.ptr + by, None)
+        return do.to_numpy((T, n_q * hd), np.float32), work.to_numpy(fill.shape, np.uint8)
+
+    got, left = run(shift)
+    assert np.array_equal(left, fill)
+    ref, left = run(0)
+    assert not np.array_equal(left, fill)
+    assert rel_err(got, ref) < 1e-5
+
+
 # ---------------------------------------------------------------- A8/A9 GQA
 @pytest.mark.parametrize("n_q,n_kv,hd,rot,gated,max_seq,start",
                          [(16, 4, 128, 32, 1, 600, (300, 511)),

@@ -92,3 +92,32 @@ def test_matmul_i8_workspace_grows_with_rows(N, K):
         sizes = [lib.qlm_matmul_i8_workspace_bytes(M, N, K, epi) for M in range(1, 301)]
         falls = [M for M in range(1, 300) if sizes[M] < sizes[M - 1]]
         assert not falls, (epi, falls)
+
+
+@pytest.mark.parametrize("max_seq", [193, 256, 257, 700, 2048, 4096, 33000])
+def test_gqa_prefill_plan_fits_the_workspace(max_seq):
+    """The split keys and the records of a prefill attention never pass the
+    workspace that the header names, at any position, row count and head
+    count; every form occurs."""
+    lib = hip.lib()
+    form, ranges, nbytes = C.c_int(), C.c_int(), C.c_size_t()
+    forms = set()
+    some = sorted({1, 2, 5, 15, 16, 17, 33, 100, 192, 193, 255, 256, 257, 290, 500, 1023, 2047,
+                   2048, max_seq // 3, max_seq // 2, max_seq - 1, max_seq})
+    for n_kv in (1, 2, 3, 4, 8, 16):
+        for G in (1, 2, 4, 8):
+            room = lib.qlm_gqa_prefill_workspace_bytes(G * n_kv, 128, max_seq)
+            for T in some:
+                for p0 in [0] + some:
+                    if T < 1 or p0 + T > max_seq:
+                        continue
+                    assert lib.qlm_gqa_prefill_plan(G * n_kv, n_kv, 128, max_seq, p0, T,
+                                                    C.byref(form), C.byref(ranges),
+                                                    C.byref(nbytes)) == 0
+                    forms.add((form.value, ranges.value > 1))
+                    assert nbytes.value <= room, (G, n_kv, p0, T)
+                    assert ranges.value >= 1
+                    assert (nbytes.value > 0) == (form.value == 3 or ranges.value > 1)
+    assert {(1, False), (2, False), (2, True)} <= forms
+    if max_seq >= 2048:
+        assert {(3, False), (3, True)} <= forms
