@@ -591,12 +591,18 @@ def cpu_baseline(model_dir, prompt, n_prompt, n_decode):
     """The reference QuickLM CPU path (its own sources, -O3 -ffast-math) on the
     same checkpoint: batched prefill of n_prompt-1 ids, then n_decode greedy
     steps; decode tokens/s as the reference CLI reports it (main.cpp:686-690).
-    One thread per physical core of this process's CPU set, pinned there."""
+    One thread per physical core of this process's CPU set, pinned there.
+    Where the reference's library is not built (its sources are not there):
+    value None and the reason."""
     from oracle.oracle import Reference
 
+    try:
+        ref = Reference("fast")
+    except FileNotFoundError as e:
+        return {"value": None, "unit": "tokens/s", "kind": "reference",
+                "reason": f"no CPU reference: {e}"}
     phys, info = host_cpus()
     os.sched_setaffinity(0, phys)
-    ref = Reference("fast")
     ref.init_threads(len(phys))
     t0 = time.perf_counter()
     m = ref.load_model(model_dir, n_prompt + n_decode + 8, "int8")
@@ -715,6 +721,9 @@ def main():
         cpu = None
         if not args.skip_cpu:
             cpu = cpu_baseline(mdir, prompts[0], args.cpu_prompt, args.cpu_decode)
+        if cpu and cpu["value"] is None:
+            log(cpu["reason"])
+        elif cpu:
             # the same prompt on the GPU: the fast-math build's stream beside it
             g, _, _ = eng.generate(prompts[:1, :args.cpu_prompt], args.cpu_decode)
             match = int(np.argmax(g[0] != cpu["tokens"])) if not np.array_equal(
@@ -855,7 +864,9 @@ def main():
                           "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                           "traffic_source": traffic_src, "bytes_per_launch": dom_b,
                           "us_per_launch": round(dom_us, 3), "launches_per_step": 36}
-    if cpu:
+    if cpu and cpu["value"] is None:
+        result["cpu_baseline"] = cpu
+    elif cpu:
         result["cpu_baseline"] = dict(cpu, sample=(
             f"4B checkpoint, batch 1: prefill (untimed) of the first {args.cpu_prompt - 1} ids "
             f"of the same 2048-token prompt, then {args.cpu_decode} greedy decode steps (timed) "

@@ -39,3 +39,17 @@ def test_pmc_record_is_this_builds():
                rec["write_kib_per_dispatch"] * rec["write_factor"]) * 1024
     assert traffic == pytest.approx(rec["traffic_bytes"], rel=1e-6)
     assert 1.0 <= rec["traffic_bytes"] / rec["bytes"] < 1.05
+
+
+def test_no_cpu_reference_is_reported(tmp_path, monkeypatch):
+    """Where the reference's library is not built the run goes on: the CPU
+    baseline says so instead of raising, and no CPU affinity is set."""
+    from oracle import oracle
+
+    monkeypatch.setattr(oracle, "REF_DIR", str(tmp_path))
+    before = os.sched_getaffinity(0)
+    cpu = bench.cpu_baseline(str(tmp_path), [1, 2, 3], 3, 1)
+    assert cpu["value"] is None
+    assert "no CPU reference" in cpu["reason"] and "not built" in cpu["reason"]
+    assert os.sched_getaffinity(0) == before
+    assert json.loads(json.dumps(cpu)) == cpu
