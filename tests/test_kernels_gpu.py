@@ -752,19 +752,21 @@ def test_deltanet_prefill_chunked(hip, orc, rng, p0, T):
         assert rel_err(out, ref) < 1e-4
 
 
-@pytest.mark.parametrize("H,T,pad,same", [(1, 16, 0, False), (3, 17, 1, False), (5, 33, 2, False),
-                                          (2, 63, 3, False), (3, 129, 1, False),
-                                          (8, 193, 4, False), (9, 255, 0, False),
-                                          (2, 320, 0, True)])
-def test_deltanet_prefill_chunked_edges(hip, rng, H, T, pad, same):
+@pytest.mark.parametrize("H,T,pad,opad,same", [
+    (1, 16, 0, 0, False), (3, 17, 1, 1, False), (5, 33, 2, 2, False), (2, 63, 3, 3, False),
+    (3, 129, 1, 1, False), (8, 193, 4, 4, False), (9, 255, 0, 0, False), (2, 320, 0, 0, True),
+    # past both thresholds (8192 row-heads: 16 rows a prep workgroup; 512
+    # workgroups: a chunk's outputs in one), 4-byte and 16-byte accesses
+    (9, 1000, 1, 1, False), (9, 1013, 2, 4, False), (11, 961, 2, 0, False)])
+def test_deltanet_prefill_chunked_edges(hip, rng, H, T, pad, opad, same):
     """Edges of the blocks of 16 rows and of the chunk ring, head counts off
-    the multiples of 8, row strides without 16-byte alignment, and a prompt of
-    one repeated row with almost no decay (every k . k is 1: the triangular
-    systems are as full as they get). 1e-4 of the row-by-row recurrence, as
-    the entry point states."""
+    the multiples of 8, row strides with and without 16-byte alignment, few
+    and many workgroups, and a prompt of one repeated row with almost no decay
+    (every k . k is 1: the triangular systems are as full as they get). 1e-4
+    of the row-by-row recurrence, as the entry point states."""
     d, p0 = 128, 4
     HD = H * d
-    ldp, ldo = 4 * HD + 2 * H + pad, HD + pad
+    ldp, ldo = 4 * HD + 2 * H + pad, HD + opad
     wt = (rng.standard_normal((4, 3 * HD)) * 0.3).astype(np.float32)
     A_log = np.log(rng.uniform(1, 16, H)).astype(np.float32)
     dtb = (rng.standard_normal(H) * 0.5 - (12 if same else 4)).astype(np.float32)
@@ -780,7 +782,7 @@ def test_deltanet_prefill_chunked_edges(hip, rng, H, T, pad, same):
     got = []
     for chunked in (False, True):
         dconv, dS, do = dev(hip, conv), dev(hip, S), dev(hip, np.full((T, ldo), 7, np.float32))
-        say("deltanet_prefill edges", H, T, pad, same, chunked)
+        say("deltanet_prefill edges", H, T, pad, opad, same, chunked)
         name = "qlm_deltanet_prefill" + ("_chunked" if chunked else "")
         tail = [work, nbytes, None] if chunked else [None]
         hip.call(name, dproj, ldp, T, dconv, *args, dS, p0, do, ldo, H, d, *tail)
@@ -834,17 +836,37 @@ def test_gqa_prefill(hip, orc, rng, n_q, n_kv, hd, rot, gated, p0, T):
     assert np.array_equal(dvc.to_numpy(vc.shape, np.float32)[:p0 + T], vref[:p0 + T])
 
 
-@pytest.mark.parametrize("n_q,n_kv,p0,T", [
-    (16, 4, 0, 192), (16, 4, 0, 193),  # the last launch of the few-key form, the first after it
-    (16, 4, 600, 5), (8, 8, 150, 60), (8, 4, 200, 45), (16, 2, 300, 33),  # key ranges merged
-    (16, 4, 70, 290), (16, 2, 0, 272),  # split planes; 19 (a middle tile) and 17 row tiles
-    (8, 4, 1, 255), (8, 8, 3, 400)])    # slots past the last in the last workgroup
-def test_gqa_prefill_split_terms(hip, orc, rng, n_q, n_kv, p0, T):
+def _prefill_form(hip, n_q, n_kv, max_seq, p0, T):
+    """The form that such a prefill attention takes and its key ranges."""
+    form, ranges, nbytes = C.c_int(), C.c_int(), C.c_size_t()
+    hip.call("qlm_gqa_prefill_plan", n_q, n_kv, 128, max_seq, p0, T, C.byref(form),
+             C.byref(ranges), C.byref(nbytes))
+    return form.value, ranges.value
+
+
+FEW, OWN, PLANES = 1, 2, 3  # few keys; split by each workgroup; split beforehand
+
+
+@pytest.mark.parametrize("n_q,n_kv,p0,T,max_seq,form,merged", [
+    # the last launch of the few-key form, the first after it
+    (16, 4, 0, 192, 700, FEW, False), (16, 4, 0, 193, 700, OWN, True),
+    (16, 4, 600, 5, 700, OWN, True), (8, 8, 150, 60, 700, OWN, True),
+    (8, 4, 200, 45, 700, OWN, True), (16, 2, 300, 33, 700, OWN, True),
+    (16, 4, 70, 290, 700, OWN, True),  # no room for planes beside the records
+    # split planes; 19 and 17 row tiles (a middle tile), 11 key blocks, the last ragged
+    (16, 4, 55, 290, 2048, PLANES, True), (16, 2, 0, 272, 700, PLANES, True),
+    # 65 row tiles, 33 key blocks, the last one ragged
+    (16, 4, 0, 1037, 2048, PLANES, False),
+    # slots past the last in the last workgroup
+    (8, 4, 1, 255, 700, OWN, True), (8, 8, 3, 400, 700, OWN, False)])
+def test_gqa_prefill_split_terms(hip, orc, rng, n_q, n_kv, p0, T, max_seq, form, merged):
     """head_dim 128 over more than a few keys (fp32 operands as three bf16
     terms): every launch form against the oracle row by row, to the fp32
     attention's bar, and an infinite V element of a key that every row sees
     (weighted by probabilities > 0: the output column is infinite)."""
-    hd, rot, max_seq, theta, gated = 128, 32, 700, 1e6, 1
+    got_form, ranges = _prefill_form(hip, n_q, n_kv, max_seq, p0, T)
+    assert (got_form, ranges > 1) == (form, merged)
+    hd, rot, theta, gated = 128, 32, 1e6, 1
     ld = n_q * 2 * hd + 2 * n_kv * hd
     qn = (rng.standard_normal(hd) * 0.02).astype(np.float32)
     kn = (rng.standard_normal(hd) * 0.02).astype(np.float32)
@@ -880,17 +902,20 @@ def test_gqa_prefill_split_terms(hip, orc, rng, n_q, n_kv, p0, T):
         assert np.array_equal(again, got)
 
 
-@pytest.mark.parametrize("n_q,n_kv,p0,T,max_seq", [
-    (16, 4, 3, 100, 700),                         # the few-key form
-    (8, 8, 150, 60, 700), (8, 4, 200, 45, 700),   # key ranges merged
-    (16, 4, 70, 290, 700), (16, 2, 37, 250, 700),  # keys split by each workgroup
-    (16, 4, 0, 304, 2048), (16, 4, 37, 600, 2048), (16, 2, 0, 272, 700)])  # split planes
-def test_gqa_prefill_values_not_finite(hip, orc, rng, n_q, n_kv, p0, T, max_seq):
+@pytest.mark.parametrize("n_q,n_kv,p0,T,max_seq,form,merged", [
+    (16, 4, 3, 100, 700, FEW, False), (8, 8, 150, 60, 700, OWN, True),
+    (8, 4, 200, 45, 700, OWN, True), (16, 4, 70, 290, 700, OWN, True),
+    (16, 2, 37, 250, 700, OWN, True), (16, 4, 37, 600, 2048, OWN, True),
+    (8, 8, 3, 400, 700, OWN, False), (16, 4, 0, 304, 2048, PLANES, True),
+    (16, 4, 0, 1037, 2048, PLANES, False), (16, 2, 0, 272, 700, PLANES, True)])
+def test_gqa_prefill_values_not_finite(hip, orc, rng, n_q, n_kv, p0, T, max_seq, form, merged):
     """An infinite or NaN V element of a prompt row reaches the rows of its
     16-row tile and later ones (a masked key of the tile is multiplied by
     probability 0), never a tile before it: those rows stay within the fp32
     attention's bar (1e-5), every other column keeps its bits. V elements at
     the top of the fp32 range keep all their bits (same bar)."""
+    got_form, ranges = _prefill_form(hip, n_q, n_kv, max_seq, p0, T)
+    assert (got_form, ranges > 1) == (form, merged)
     hd, rot, theta, gated = 128, 32, 1e6, 1
     ld, kv = n_q * 2 * hd + 2 * n_kv * hd, n_kv - 1
     qn = (rng.standard_normal(hd) * 0.02).astype(np.float32)
@@ -938,7 +963,8 @@ def test_gqa_prefill_values_not_finite(hip, orc, rng, n_q, n_kv, p0, T, max_seq)
         assert rel_err(got[t:, heads, c] * scale, ref[t:, heads, c] * scale) < 1e-5
 
 
-@pytest.mark.parametrize("n_q,n_kv,p0,T", [(16, 4, 600, 5), (16, 4, 20, 320), (8, 8, 150, 60)])
+@pytest.mark.parametrize("n_q,n_kv,p0,T", [(16, 4, 600, 5), (16, 4, 20, 320), (8, 8, 150, 60),
+                                           (32, 4, 0, 1057)])
 @pytest.mark.parametrize("shift", [4, 8])
 def test_gqa_prefill_workspace_alignment(hip, orc, rng, n_q, n_kv, p0, T, shift):
     """A workspace that is not 16-byte aligned is accepted and left unused:
