@@ -706,11 +706,6 @@ __device__ __forceinline__ f32x4 mfma_bf16(pf_u32x4 a, pf_u32x4 b, f32x4 c) {
 // 2^x for x <= 0 by v_exp_f32 (1 ulp)
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
-__device__ __forceinline__ bool finite4(f32x4 v) {
-    const f32x4 z = v * 0.0f;  // NaN for one that is not
-    return (z[0] + z[1]) + (z[2] + z[3]) == 0.0f;
-}
-
 // ---- the fp32 form: 16 query rows x 16 keys on v_mfma_f32_16x16x4f32 ----
 //
 // A lane l: row l % 16, k l / 16; B lane l: k l / 16, column l % 16; D lane l:
@@ -1118,24 +1113,17 @@ __global__ __launch_bounds__(PfShape<G>::NTH, 2) void k_attn_pf(
                 o[r][c >> 2][c & 3] = o[r][c >> 2][c & 3] * f0 + mg[r][at * RS + c] * f1;
         }
     }
-    // where elements 16 c + 4 qd .. + 3 of row t go (record or output), and what
-    // becomes of them on the way
+    // row t's record or output, and the elements 16 c + 4 qd .. + 3 of an output
     auto record = [&](int t) {
         return work +
                (((size_t)t * (gridDim.y * G) + h) * gridDim.z + blockIdx.z) * (HD + 4);
     };
-    auto place = [&](int t, int c) {
-        return reinterpret_cast<f32x4*>(work ? record(t) + 4 + 16 * c + 4 * qd
-                                             : out + (size_t)t * ldo + (size_t)h * HD + 16 * c +
-                                                   4 * qd);
-    };
+    auto output = [&](int t) { return out + (size_t)t * ldo + (size_t)h * HD; };
     auto gate = [&](int t, int c, f32x4 y) {
-        if (gated && !work) {
-            const f32x4 gg = *reinterpret_cast<const f32x4*>(
-                qkv + (size_t)t * ldq + (size_t)h * qhs + HD + 16 * c + 4 * qd);
+        const f32x4 gg = *reinterpret_cast<const f32x4*>(qkv + (size_t)t * ldq + (size_t)h * qhs +
+                                                         HD + 16 * c + 4 * qd);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) y[i] /= 1.0f + expf(-gg[i]);
-        }
+        for (int i = 0; i < 4; ++i) y[i] /= 1.0f + expf(-gg[i]);
         return y;
     };
     bool odd[2] = {false, false};
@@ -1143,28 +1131,39 @@ __global__ __launch_bounds__(PfShape<G>::NTH, 2) void k_attn_pf(
     for (int r = 0; r < 2; ++r) {
         const int tq = t0[r] + n;
         if (last[r] < kbeg || tq >= T) continue;
-        float f;
+        f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};  // NaN where an output is not finite
         if (work) {
             // the record's maximum is in natural units; what its rounding
             // changes goes into l and o
             const float mr = m[r] * 0.69314718f;
             float e = fmaf(-mr, 1.44269502f, m[r]);
             e = m[r] == -INFINITY ? 0.0f : fmaf(-mr, 1.92596303e-8f, e);
-            f = exp2_fast(e);
+            const float f = exp2_fast(e);
+            float* rec = record(tq);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const f32x4 y = o[r][c] * f;
+                *reinterpret_cast<f32x4*>(rec + 4 + 16 * c + 4 * qd) = y;
+                z += y * 0.0f;
+            }
             if (qd == 0) {
-                record(tq)[0] = mr;
-                record(tq)[1] = l[r] * f;
+                rec[0] = mr;
+                rec[1] = l[r] * f;
             }
         } else {
-            f = 1.0f / l[r];
-        }
+            float* dst = output(tq);
+            const float inv = 1.0f / l[r];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const f32x4 y = gate(tq, c, o[r][c] * f);
-            *place(tq, c) = y;
-            odd[r] |= !finite4(y);
+            for (int c = 0; c < 8; ++c) {
+                f32x4 y = o[r][c] * inv;
+                if (gated) y = gate(tq, c, y);
+                *reinterpret_cast<f32x4*>(dst + 16 * c + 4 * qd) = y;
+                z += y * 0.0f;
+            }
         }
+        odd[r] = (z[0] + z[1]) + (z[2] + z[3]) != 0.0f;
     }
+    if (__builtin_expect(!__any(odd[0] || odd[1]), 1)) return;
 #pragma unroll 1
     for (int r = 0; r < 2; ++r) {
         const bool mine = r ? odd[1] : odd[0];
@@ -1176,13 +1175,15 @@ __global__ __launch_bounds__(PfShape<G>::NTH, 2) void k_attn_pf(
                                    qscale * 0.69314718f);
         if (!mine) continue;
         const float f = work ? expf(a.m - (r ? m[1] : m[0]) * 0.69314718f) : 1.0f / a.l;
+        float* dst = work ? record(tq) + 4 : output(tq);
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            f32x4 y = *place(tq, c);
-            const f32x4 z = gate(tq, c, a.o[c] * f);
+            f32x4* at = reinterpret_cast<f32x4*>(dst + 16 * c + 4 * qd);
+            f32x4 y = *at, again = a.o[c] * f;
+            if (gated && !work) again = gate(tq, c, again);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) y[i] = y[i] * 0.0f == 0.0f ? y[i] : z[i];
-            *place(tq, c) = y;
+            for (int i = 0; i < 4; ++i) y[i] = y[i] * 0.0f == 0.0f ? y[i] : again[i];
+            *at = y;
         }
     }
 }
