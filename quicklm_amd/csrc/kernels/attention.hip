@@ -601,10 +601,12 @@ __global__ __launch_bounds__(kThreads) void k_gqa_prep_rows(
 //
 // Bound by the matrix cores and the vector ALUs in turn (the waves of a
 // workgroup are at the products, then at the softmax, together): 2047 rows
-// 131 us at ~35% of the bf16 peak counting all six products, 2048 rows after
-// 2048 keys 300 us. The fp32 form, one 16-row tile a workgroup, took 363 and
+// 136 us at ~30% of the bf16 peak counting all six products, 2048 rows after
+// 2048 keys 311 us (medians of traces). The fp32 form, one 16-row tile a workgroup, took 363 and
 // 787 us: 16x the matrix time a product, its longest tile alone 128 or 256
-// steps of 16 keys; 5 rows after 600 keys 71 us, now 13 and a 4 us merge.
+// steps of 16 keys; 5 rows after 600 keys 71 us, now 16 and a 4 us merge. The
+// form that splits its own keys (up to 4 heads) is out of registers: 43 of them
+// go through scratch.
 //
 // Row tiles of 16 are paired first with last (tile a with nt - 1 - a), so
 // every slot of two tiles attends to about the same number of keys. A
